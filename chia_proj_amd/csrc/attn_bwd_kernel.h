@@ -26,8 +26,23 @@
 //     every query head of the group (GQA): S = Q K^T and dP = dO V^T with K, V
 //     in registers (lane = key), dV^T += dO^T P and dK^T += Q^T dS with Q and
 //     dO read transposed.
-// Tiles are 64 rows, DMA'd HBM -> LDS as in the forward (one swizzle for both
-// the row and the transposed reads), three LDS stages, one barrier per tile.
+// Tiles are 64 rows (32 in dK/dV at head_dim 128), DMA'd HBM -> LDS as in the
+// forward (one swizzle for both the row and the transposed reads), three LDS
+// stages at head_dim 64 and two at 128, one barrier per tile.
+//
+// Both kernels keep two wavefronts on every SIMD (two workgroups per CU): one
+// alone waits out every dependent MFMA, exponential and LDS read.  At head_dim
+// 128 that is a budget of 256 registers and 80 KB of LDS per workgroup:
+//   * dQ fits it with two stages of 64-key tiles (64 KB);
+//   * dK/dV holds 128 accumulators, so its K fragments stay in LDS (32 KB, read
+//     beside the Q rows) and only V's in registers, its tiles are 32 rows (two
+//     stages, 33 KB), and a scheduling barrier every four k-steps bounds the
+//     fragments in flight (without it the compiler hoists them and spills
+//     8-24 registers).
+// Against one wavefront per SIMD (three 64-row stages, 440 registers), dQ +
+// dK/dV: causal ALiBi B2 H32 S2048 D128 392 -> 268 us, full sigmoid B2 H16
+// S4096 D128 1452 -> 961 us, window 256 B4 H16 S2048 D128 188 -> 131 us;
+// gradients bit-identical.
 #pragma once
 #include "attn_fwd_kernel.h"
 
@@ -44,6 +59,11 @@ __device__ __forceinline__ void dma4s(const void* sbase, uint32_t voff, uint32_t
   const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
   const uint64_t u = ((uint64_t)hi << 32) | (uint64_t)lo;
   asm volatile("global_load_lds_dword %0, %1" ::"v"(voff), "s"(u), "{m0}"(lds_base) : "memory");
+}
+
+// A wavefront-uniform float in a scalar register.
+__device__ __forceinline__ float uniform_f(float x) {
+  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x)));
 }
 
 struct BwdParams {
@@ -175,17 +195,17 @@ __device__ __forceinline__ ScoreGrad<NORM, ALIBI, SOFTCAP> score_consts(const Bw
   return f;
 }
 
-// One 64-row tile of a [S, D] bf16 tensor (row stride rs elements, rows from
+// One ROWS-row tile of a [S, D] bf16 tensor (row stride rs elements, rows from
 // `row` of the residue's sub-sequence, clamped to S - 1) into LDS at `dst`:
 // row r, 16-byte chunk c lands in slot k_slot<D>(r, c), which keeps both the
 // row reads and the transposed reads of the tile free of bank conflicts.
 // Wavefront w of NW moves
 // chunks [(n NW + w) 64, +64) for n < NDMA.
-template <int D, int NW>
+template <int D, int NW, int ROWS = 64>
 __device__ __forceinline__ void dma_rows(const uint16_t* base, int64_t rs, int row, int S, char* dst, int wave,
                                          int lane) {
   constexpr int DQ = D / 8;
-  constexpr int NDMA = 64 * DQ / (NW * 64);
+  constexpr int NDMA = ROWS * DQ / (NW * 64);
   const uint16_t* src = base + (int64_t)row * rs;
 #pragma unroll
   for (int n = 0; n < NDMA; ++n) {
@@ -197,13 +217,13 @@ __device__ __forceinline__ void dma_rows(const uint16_t* base, int64_t rs, int r
 }
 
 // dma_rows with its per-lane offsets computed once for a fixed row stride: a
-// tile whose 64 rows lie inside the sub-sequence adds only its uniform row
+// tile whose ROWS rows lie inside the sub-sequence adds only its uniform row
 // base, a 32 x 32 -> 64-bit product (rows are non-negative and a row step is
 // below 2^25 elements, so its byte count fits 32 bits); the last tile, whose
 // rows past the end are clamped, takes dma_rows.
-template <int D, int NW>
+template <int D, int NW, int ROWS = 64>
 struct RowDma {
-  static constexpr int DQ = D / 8, NDMA = 64 * DQ / (NW * 64);
+  static constexpr int DQ = D / 8, NDMA = ROWS * DQ / (NW * 64);
   uint32_t off[NDMA];
   uint32_t row_bytes;
   __device__ RowDma(int64_t rs, int wave, int lane) : row_bytes(2u * (uint32_t)rs) {
@@ -215,12 +235,12 @@ struct RowDma {
     }
   }
   __device__ void operator()(const uint16_t* base, int64_t rs, int row, int S, char* dst, int wave, int lane) const {
-    if (row + 64 <= S) {
+    if (row + ROWS <= S) {
       const uint16_t* src = (const uint16_t*)((const char*)base + (uint64_t)(uint32_t)row * row_bytes);
 #pragma unroll
       for (int n = 0; n < NDMA; ++n) dma16s(src, off[n], lds_addr(dst + (n * NW + wave) * 1024));
     } else {
-      dma_rows<D, NW>(base, rs, row, S, dst, wave, lane);
+      dma_rows<D, NW, ROWS>(base, rs, row, S, dst, wave, lane);
     }
   }
 };
@@ -259,10 +279,10 @@ __device__ __forceinline__ float half_row_dot(const bf16x8_t* x, const bf16x8_t*
 
 // ---- dQ ------------------------------------------------------------------------
 template <int D, int NORM, bool ALIBI, bool SOFTCAP>
-__global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_dq_kernel(const BwdParams p) {
+__global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(const BwdParams p) {
   constexpr int NW = 4, BN = 64, KB = BN / 32, DK = D / 16, DB = D / 32;
   constexpr int RP = 2 * D, T_BYTES = BN * RP, STAGE_BYTES = 2 * T_BYTES;
-  constexpr int NS = 3;
+  constexpr int NS = D == 64 ? 3 : 2;
   __shared__ __attribute__((aligned(1024))) char lds[NS * STAGE_BYTES];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -479,15 +499,18 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_dq_kernel(const
 // per-head scales), so c1 multiplies each score; otherwise it multiplies dK
 // once at the store.
 template <int D, int NORM, bool ALIBI, bool SOFTCAP, bool HEAD_C1>
-__global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_dkdv_kernel(const BwdParams p) {
-  constexpr int NW = 4, BM = 64, QB = BM / 32, DK = D / 16, DB = D / 32;
+__global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(const BwdParams p) {
+  constexpr bool kKLds = D == 128;  // K fragments read from LDS, not kept in registers
+  constexpr int NW = 4, BM = D == 64 ? 64 : 32, QB = BM / 32, DK = D / 16, DB = D / 32;
   constexpr int RP = 2 * D, T_BYTES = BM * RP;
-  // stage: Q tile, dO tile, then (softmax) the 64 rows' lse log2 e and -delta
+  // stage: Q tile, dO tile, then (softmax) the BM rows' lse log2 e and -delta
   constexpr bool kStats = NORM == NORM_SOFTMAX;
-  constexpr int STAGE_BYTES = 2 * T_BYTES + (kStats ? 512 : 0);
-  constexpr int NS = 3;
+  constexpr int STAGE_BYTES = 2 * T_BYTES + (kStats ? 8 * BM : 0);
+  constexpr int NS = D == 64 ? 3 : 2;
   constexpr int kMaxGroup = 256;  // query heads per K/V head staged in LDS
+  constexpr int KW_BYTES = 32 * RP;  // a wavefront's K rows
   __shared__ __attribute__((aligned(1024))) char lds[NS * STAGE_BYTES];
+  __shared__ __attribute__((aligned(1024))) char lds_k[kKLds ? NW * KW_BYTES : 16];
   __shared__ float head_c[2 * kMaxGroup];  // per query head of the group: c1, ALiBi slope
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -535,19 +558,21 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_dkdv_kernel(con
   __syncthreads();
   // ds leaves the score step without c1: applied to dK at the store when the
   // group shares one scale, else per score
-  const float c1u = HEAD_C1 ? 1.0f : head_c[0];
+  const float c1u = HEAD_C1 ? 1.0f : (D == 64 ? head_c[0] : uniform_f(head_c[0]));
 
-  // this wavefront's 32 keys: K and V as MFMA B operands (lane = key)
+  // this wavefront's 32 keys: K and V as MFMA B operands (lane = key); K rows
+  // kept in LDS are read by the wavefront that loads them, after its first wait
   const int key0 = blk * 128 + 32 * wave;
   const int j = key0 + lq;
   const bool okj = j < g.S;
-  bf16x8_t kf[DK], vf[DK];
+  bf16x8_t kf[kKLds ? 1 : DK], vf[DK];
+  if constexpr (kKLds) dma_rows<D, 1, 32>(kh, krs, imin32(key0, g.S - 1), g.S, lds_k + wave * KW_BYTES, 0, lane);
   {
     const uint16_t* ks = kh + (int64_t)(okj ? j : 0) * krs + 8 * lh;
     const uint16_t* vs = vh + (int64_t)(okj ? j : 0) * vrs + 8 * lh;
 #pragma unroll
     for (int kk = 0; kk < DK; ++kk) {
-      kf[kk] = __builtin_bit_cast(bf16x8_t, *(const u32x4_t*)(ks + 16 * kk));
+      if constexpr (!kKLds) kf[kk] = __builtin_bit_cast(bf16x8_t, *(const u32x4_t*)(ks + 16 * kk));
       vf[kk] = __builtin_bit_cast(bf16x8_t, *(const u32x4_t*)(vs + 16 * kk));
     }
   }
@@ -603,7 +628,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_dkdv_kernel(con
   // Scalar work per tile is kept small: the stage is a wrapping counter, the
   // class of a row tile comes from the wavefront's two row spans (mask.h), and
   // the DMA's per-lane offsets are fixed once.
-  const RowDma<D, NW> qdma(qrs, wave, lane), dodma(dors, wave, lane);
+  const RowDma<D, NW, BM> qdma(qrs, wave, lane), dodma(dors, wave, lane);
   const RowRanges<BM> rr(g, wvalid, kc, kd);
   uint32_t st_cur = 0;
   auto issue = [&](uint32_t stage) {
@@ -612,19 +637,22 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_dkdv_kernel(con
     qdma(dc.qb, qrs, i0, g.S, st, wave, lane);
     dodma(dc.dob, dors, i0, g.S, st + T_BYTES, wave, lane);
     if constexpr (kStats) {
-      // wavefront w moves 32 floats: lse log2 e rows [32 w, +32) (w < 2), or
-      // -delta rows [32 (w - 2), +32); the stats rows are padded to 64
-      const float* src = dc.sb + (wave >= 2 ? plane : 0) + i0 + 32 * (wave & 1);
-      if (lane < 32) dma4s(src, (uint32_t)(4 * lane), lds_addr(st + 2 * T_BYTES + 128 * wave));
+      // wavefront w moves BM / 2 floats: lse log2 e rows [w BM / 2, +BM / 2) (w < 2),
+      // or -delta rows [(w - 2) BM / 2, +BM / 2); the stats rows are padded to 64
+      const float* src = dc.sb + (wave >= 2 ? plane : 0) + i0 + BM / 2 * (wave & 1);
+      if (lane < BM / 2) dma4s(src, (uint32_t)(4 * lane), lds_addr(st + 2 * T_BYTES + 2 * BM * wave));
     }
     advance(dc);
   };
-  constexpr int NDMA2 = 2 * (64 * (D / 8) / (NW * 64)) + (kStats ? 1 : 0);
+  constexpr int NDMA2 = 2 * (BM * (D / 8) / (NW * 64)) + (kStats ? 1 : 0);
   int dma_next = 0;
   for (; dma_next < NS - 1 && dma_next < ntiles; ++dma_next) issue((uint32_t)dma_next);
   // K and V in registers before the loop (see the dQ kernel)
 #pragma unroll
-  for (int kk = 0; kk < DK; ++kk) asm volatile("" : "+v"(kf[kk]), "+v"(vf[kk]));
+  for (int kk = 0; kk < DK; ++kk) {
+    if constexpr (!kKLds) asm volatile("" : "+v"(kf[kk]));
+    asm volatile("" : "+v"(vf[kk]));
+  }
 
   typedef short i16x8_t __attribute__((ext_vector_type(8)));
   for (int it = 0; it < ntiles; ++it) {
@@ -647,8 +675,10 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_dkdv_kernel(con
     if (i0 + BM > g.S) cls = TILE_PARTIAL;
     constexpr bool kSeed = ALIBI && !SOFTCAP;  // as in the dQ kernel
     ScoreGrad<NORM, ALIBI && !kSeed, SOFTCAP> sg = score_consts<NORM, ALIBI && !kSeed, SOFTCAP>(p);
-    sg.set_head(head_c[hq - hkv * p.G], head_c[kMaxGroup + hq - hkv * p.G]);
-    const float* st_stats = (const float*)(St + 2 * T_BYTES);  // [64] lse log2 e, then [64] -delta
+    const float hc1 = head_c[hq - hkv * p.G], hsl = head_c[kMaxGroup + hq - hkv * p.G];
+    if constexpr (D == 64) sg.set_head(hc1, hsl);
+    else sg.set_head(uniform_f(hc1), uniform_f(hsl));  // (no vector register to spare)
+    const float* st_stats = (const float*)(St + 2 * T_BYTES);  // [BM] lse log2 e, then [BM] -delta
 
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
@@ -656,11 +686,15 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_dkdv_kernel(con
       // log2 e, and -delta as the dP accumulator's seed
       const int ibase = i0 + 32 * qb + 4 * lh;
       f32x4_t l4[4], d4[4];
+      auto read_lse = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int gq = 0; gq < 4; ++gq) l4[gq] = *(const f32x4_t*)(st_stats + 32 * qb + 4 * lh + 8 * gq);
+      };
       if constexpr (kStats) {
+        if constexpr (D == 64) read_lse();  // (head_dim 128: no registers for them until the scores are done)
 #pragma unroll
         for (int gq = 0; gq < 4; ++gq) {
-          l4[gq] = *(const f32x4_t*)(st_stats + 32 * qb + 4 * lh + 8 * gq);
-          d4[gq] = *(const f32x4_t*)(st_stats + 64 + 32 * qb + 4 * lh + 8 * gq);
+          d4[gq] = *(const f32x4_t*)(st_stats + BM + 32 * qb + 4 * lh + 8 * gq);
         }
       }
       f32x16_t sacc, pacc;
@@ -678,9 +712,13 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_dkdv_kernel(con
       for (int kk = 0; kk < DK; ++kk) {
         const bf16x8_t a = *(const bf16x8_t*)(St + 32 * qb * RP + (k_lane ^ (32 * kk)));
         const bf16x8_t ad = *(const bf16x8_t*)(St + T_BYTES + 32 * qb * RP + (k_lane ^ (32 * kk)));
-        sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, kf[kk], sacc, 0, 0, 0);
+        const bf16x8_t kb = kKLds ? *(const bf16x8_t*)(lds_k + wave * KW_BYTES + (k_lane ^ (32 * kk))) : kf[kKLds ? 0 : kk];
+        sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, kb, sacc, 0, 0, 0);
         pacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ad, vf[kk], pacc, 0, 0, 0);
+        // head_dim 128: at most four steps' fragments in flight (more spill)
+        if constexpr (D == 128) if ((kk & 3) == 3) __builtin_amdgcn_sched_barrier(0);
       }
+      if constexpr (kStats && D == 128) read_lse();
       float pv[16], dsv[16];
 #pragma unroll
       for (int e = 0; e < 16; ++e) {

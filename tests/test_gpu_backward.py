@@ -108,6 +108,18 @@ def test_backward_edge_cases(name, B, H, Hkv, S, D, kw):
     _check(name, grads, refs)
 
 
+@pytest.mark.parametrize("S", [1, 31, 32, 33, 96, 127, 129, 161])
+@pytest.mark.parametrize("kw", [dict(causal=True), dict(causal=False, window=20),
+                                dict(causal=True, softcap=15.0, alibi_slopes=[0.3, 0.1, 0.05, 0.02])],
+                         ids=["causal", "local20", "softcap_alibi"])
+def test_backward_d128_row_tile_edges(S, kw):
+    """Head dim 128 around the 32-row tiles and 128-key blocks of dK/dV, two heads per K/V head."""
+    _say(f"[bwd] d128 edge S={S} {kw}")
+    q, k, v, do = _draw(1, 4, 2, S, 128, 900 + S)
+    _, grads = _run(q, k, v, do, lambda a, b, c: attention(a, b, c, **kw))
+    _check(f"S={S} {kw}", grads, attention_grad_ref(q, k, v, do, **kw))
+
+
 def test_backward_causal_s2048_sampled_heads():
     """B2 H4 S2048 D64 causal softmax: the full kernel grid, two heads checked."""
     _say("[bwd] causal S2048")

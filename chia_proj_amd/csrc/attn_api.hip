@@ -316,7 +316,7 @@ extern "C" int chia_attn_fwd_lse(const chia_attn_args* a, float* lse, void* stre
 
 namespace {
 constexpr int kBwdMaxGroup = 256;  // query heads per K/V head the dK/dV kernel stages
-constexpr int kBwdBlock = 128;     // rows (dQ) or keys (dK/dV) per workgroup
+constexpr int kBwdBlock = 128;     // rows per dQ workgroup (dK/dV: 32 keys per key wavefront)
 
 // Rows of the stats workspace per (b, h, residue): residue 0's length padded
 // to the 64-row tiles the dK/dV kernel reads whole.
@@ -328,12 +328,63 @@ int64_t bwd_workspace(const chia_attn_args* a) {
   return 2 * a->batch * a->heads * (int64_t)num_residues(m) * stats_rows(m) * (int64_t)sizeof(float);
 }
 
-hipError_t launch(BwdKernelFn fn, int64_t grid, const BwdParams& p, hipStream_t stream) {
+// Which workgroup shape the dK/dV kernel takes (kDkdvSplit), by an estimate of
+// the launch's time on 256 CUs.  The unit is one (128-key, row tile) step on a
+// fully occupied CU.  A launch of n workgroups of KW key wavefronts and QG
+// groups, whose walks have the longest length `l`, is bound by
+//   * the work of all of them spread evenly, or
+//   * the k-th round of CUs: k (P_k) where P_k is about the length of walk
+//     number 256 (k - 1) in falling order (the lengths taken as falling
+//     linearly from the longest), a workgroup of four wavefronts that is alone
+//     on its CU running at 1 / 1.3 of the CU's rate,
+// times what the split costs per step (1.05 for two groups: one workgroup per
+// CU instead of two, so start and end overlap less; 1.6 for four: each Q / dO
+// tile serves 64 keys instead of 128), plus 4 steps per round of start-up and
+// 2 more for adding the groups' sums.  The constants fit 110 drawn shapes (1-4
+// sequences of 128-4096 tokens, 1-32 K/V heads, every mask): within 0.3 % of
+// the best shape on average, never more than 3 % above {4, 1}, which by itself
+// was 21 % above the best (up to 1.9x: B1 H32/8 S3000 D128 causal, dQ + dK/dV
+// 561 us against 424 {4, 2} and 305 {2, 4}; B4 H16 S4096 D64 490 against 567
+// and 657).
+int pick_dkdv_split(const MaskSpec& m, int64_t slices, int64_t group, int32_t row_tile) {
+  const MaskGeom g = residue_geom(m, 0);
+  const int32_t nblk = (g.S + kBwdBlock - 1) / kBwdBlock;
+  // walks of the first, the middle and the last key block
+  auto walk = [&](int32_t blk) {
+    const RowSpan r = query_range(g, blk * kBwdBlock, imin32(blk * kBwdBlock + kBwdBlock - 1, g.S - 1));
+    return (double)group * (r.hi / row_tile - r.lo / row_tile + 1);
+  };
+  const double w0 = walk(0), w1 = walk(nblk / 2), w2 = walk(nblk - 1);
+  const double longest = std::fmax(w0, std::fmax(w1, w2)), mean = 0.25 * (w0 + 2.0 * w1 + w2);
+  constexpr double kPerStep[kDkdvSplits] = {1.0, 1.05, 1.6};
+  int best = 0;
+  double best_cost = 0.0;
+  for (int s = 0; s < kDkdvSplits; ++s) {
+    const DkdvSplit sp = kDkdvSplit[s];
+    const double unit = sp.kw / 4.0, n = (double)slices * nblk / unit;
+    const double alone = sp.kw * sp.qg == 8 ? 1.0 : 1.3;
+    double t = n * mean * unit / kCUs;
+    for (int k = 1; k <= 8 && (k - 1) * kCUs < n; ++k) {
+      const double len = longest - 2.0 * (longest - mean) * ((k - 1) * kCUs / n);
+      t = std::fmax(t, k * len * unit * (k == 1 ? alone : 1.0));
+    }
+    const double rounds = std::fmax(1.0, n / (sp.qg == 1 ? 2 * kCUs : kCUs));
+    const double cost = kPerStep[s] * t + (sp.qg == 1 ? 4.0 : 6.0) * rounds;
+    if (s == 0 || cost < best_cost) {
+      best = s;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
+hipError_t launch(BwdKernelFn fn, int64_t grid, int threads, const BwdParams& p, hipStream_t stream) {
   if (grid <= 0) return hipSuccess;
   BwdParams q = p;
   q.n_wg = (int32_t)grid;
   void* kargs[] = {&q};
-  const hipError_t err = hipLaunchKernel(reinterpret_cast<const void*>(fn), dim3((unsigned)grid), dim3(256), kargs, 0, stream);
+  const hipError_t err =
+      hipLaunchKernel(reinterpret_cast<const void*>(fn), dim3((unsigned)grid), dim3(threads), kargs, 0, stream);
   return err != hipSuccess ? err : hipGetLastError();
 }
 }  // namespace
@@ -472,7 +523,6 @@ int launch_bwd(const chia_attn_bwd_args* ba, void* stream, bool noalloc) {
   p.post_scale = a->post_scale;
 
   const int64_t g_dq = a->batch * a->heads * p.residues * (int64_t)p.n_blk;
-  const int64_t g_dkdv = a->batch * hkv * p.residues * (int64_t)p.n_blk;
   if (g_dq >= ((int64_t)1 << 31)) return CHIA_ATTN_ERR_SHAPE;
 
   const bool alibi = a->alibi_slopes != nullptr, softcap = a->softcap > 0.f;
@@ -489,11 +539,16 @@ int launch_bwd(const chia_attn_bwd_args* ba, void* stream, bool noalloc) {
     p.div_hx = make_udiv(on ? p.rank_hx : 1);
   };
   rank_for(a->batch * a->heads * p.residues);
-  err = launch(ks.dq, g_dq, p, s);
+  err = launch(ks.dq, g_dq, 256, p, s);
   rank_for(a->batch * hkv * p.residues);
+  const int split = pick_dkdv_split(p.mask, a->batch * hkv * p.residues, G, a->head_dim == 64 ? 64 : 32);
+  const DkdvSplit sp = kDkdvSplit[split];
+  p.n_blk = (residue_geom(p.mask, 0).S + 32 * sp.kw - 1) / (32 * sp.kw);
+  p.div_blk = make_udiv(p.n_blk);
   // a group whose query heads differ in scale takes c1 per score
-  const BwdKernelFn dkdv = G > 1 && a->head_scale ? ks.dkdv_head_c1 : ks.dkdv;
-  if (err == hipSuccess) err = launch(dkdv, g_dkdv, p, s);
+  const BwdKernelFn dkdv = ks.dkdv[split][G > 1 && a->head_scale ? 1 : 0];
+  if (err == hipSuccess)
+    err = launch(dkdv, a->batch * hkv * p.residues * (int64_t)p.n_blk, 64 * sp.kw * sp.qg, p, s);
   return err == hipSuccess ? CHIA_ATTN_OK : (int)err;
 }
 }  // namespace

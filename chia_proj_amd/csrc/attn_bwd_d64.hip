@@ -4,10 +4,21 @@
 
 namespace chia {
 
+template <int NORM, bool AL, bool SC, int SPLIT>
+static void set_dkdv(BwdKernels& k) {
+  constexpr int KW = kDkdvSplit[SPLIT].kw, QG = kDkdvSplit[SPLIT].qg;
+  k.dkdv[SPLIT][0] = attn_bwd_dkdv_kernel<64, NORM, AL, SC, false, KW, QG>;
+  k.dkdv[SPLIT][1] = attn_bwd_dkdv_kernel<64, NORM, AL, SC, true, KW, QG>;
+}
+
 template <int NORM, bool AL, bool SC>
 static BwdKernels bwd_inst() {
-  return BwdKernels{attn_bwd_dq_kernel<64, NORM, AL, SC>, attn_bwd_dkdv_kernel<64, NORM, AL, SC, false>,
-                    attn_bwd_dkdv_kernel<64, NORM, AL, SC, true>};
+  BwdKernels k;
+  k.dq = attn_bwd_dq_kernel<64, NORM, AL, SC>;
+  set_dkdv<NORM, AL, SC, 0>(k);
+  set_dkdv<NORM, AL, SC, 1>(k);
+  set_dkdv<NORM, AL, SC, 2>(k);
+  return k;
 }
 
 BwdKernels select_bwd_kernels_d64(int norm, bool alibi, bool softcap) {

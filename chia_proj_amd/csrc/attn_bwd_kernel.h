@@ -224,11 +224,16 @@ __device__ __forceinline__ void dma_rows(const uint16_t* base, int64_t rs, int r
 template <int D, int NW, int ROWS = 64>
 struct RowDma {
   static constexpr int DQ = D / 8, NDMA = ROWS * DQ / (NW * 64);
-  uint32_t off[NDMA];
+  // The swizzle has a period of 16 rows, so loads 16 rows apart share one
+  // offset: with two wavefronts (twice the loads each) only the distinct ones
+  // are kept and the rest is added to the uniform base.
+  static constexpr int RS = NW * 64 / DQ;  // rows per load
+  static constexpr int ND = NW == 4 || RS * NDMA <= 16 ? NDMA : (RS >= 16 ? 1 : 16 / RS);
+  uint32_t off[ND];
   uint32_t row_bytes;
   __device__ RowDma(int64_t rs, int wave, int lane) : row_bytes(2u * (uint32_t)rs) {
 #pragma unroll
-    for (int n = 0; n < NDMA; ++n) {
+    for (int n = 0; n < ND; ++n) {
       const int pos = (n * NW + wave) * 64 + lane;
       const int r = pos / DQ, slot = pos % DQ;
       off[n] = (uint32_t)r * row_bytes + 16 * k_slot<D>(r, slot);
@@ -238,7 +243,9 @@ struct RowDma {
     if (row + ROWS <= S) {
       const uint16_t* src = (const uint16_t*)((const char*)base + (uint64_t)(uint32_t)row * row_bytes);
 #pragma unroll
-      for (int n = 0; n < NDMA; ++n) dma16s(src, off[n], lds_addr(dst + (n * NW + wave) * 1024));
+      for (int n = 0; n < NDMA; ++n)
+        dma16s((const char*)src + (uint64_t)(uint32_t)(n / ND * ND * RS) * row_bytes, off[n % ND],
+               lds_addr(dst + (n * NW + wave) * 1024));
     } else {
       dma_rows<D, NW, ROWS>(base, rs, row, S, dst, wave, lane);
     }
@@ -253,10 +260,19 @@ __device__ __forceinline__ uint32_t stage_behind(uint32_t cur) {
   return cur == 0 ? NS - 1 : cur - 1;
 }
 
+// Workgroup shapes of the dK/dV kernel: key wavefronts (32 keys each) times
+// query groups that split the walk over the query tiles.
+constexpr int kDkdvSplits = 3;
+struct DkdvSplit {
+  int kw, qg;
+};
+constexpr DkdvSplit kDkdvSplit[kDkdvSplits] = {{4, 1}, {4, 2}, {2, 4}};
+
 // Kernel set of one (head_dim, normaliser, ALiBi, softcap) instantiation.
 using BwdKernelFn = void (*)(BwdParams);
 struct BwdKernels {
-  BwdKernelFn dq, dkdv, dkdv_head_c1;  // dkdv_head_c1: a group's heads differ in scale
+  BwdKernelFn dq;
+  BwdKernelFn dkdv[kDkdvSplits][2];  // [split][1: a K/V group's heads differ in scale]
 };
 
 // do . o over the 8 DK bf16 values of one lane's half row (chunks 16 kk + 8 lh
@@ -498,23 +514,31 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(const BwdParams p) 
 // HEAD_C1: the query heads of a K/V group differ in score scale (GQA with
 // per-head scales), so c1 multiplies each score; otherwise it multiplies dK
 // once at the store.
-template <int D, int NORM, bool ALIBI, bool SOFTCAP, bool HEAD_C1>
-__global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(const BwdParams p) {
+// KW: key wavefronts, 32 keys each.  QG: query groups of KW wavefronts that
+// split the walk over the query tiles (tile t belongs to group t % QG, each
+// group with its own LDS stages) and add their sums at the end: for grids too
+// small to fill the chip, or whose longest walk would outlast the rest.
+template <int D, int NORM, bool ALIBI, bool SOFTCAP, bool HEAD_C1, int KW, int QG>
+__global__ __launch_bounds__(64 * KW * QG, 2) void attn_bwd_dkdv_kernel(const BwdParams p) {
   constexpr bool kKLds = D == 128;  // K fragments read from LDS, not kept in registers
-  constexpr int NW = 4, BM = D == 64 ? 64 : 32, QB = BM / 32, DK = D / 16, DB = D / 32;
+  constexpr int NW = KW, BM = D == 64 ? 64 : 32, QB = BM / 32, DK = D / 16, DB = D / 32;
+  constexpr int BK = 32 * KW;  // keys per workgroup
   constexpr int RP = 2 * D, T_BYTES = BM * RP;
   // stage: Q tile, dO tile, then (softmax) the BM rows' lse log2 e and -delta
   constexpr bool kStats = NORM == NORM_SOFTMAX;
   constexpr int STAGE_BYTES = 2 * T_BYTES + (kStats ? 8 * BM : 0);
-  constexpr int NS = D == 64 ? 3 : 2;
+  constexpr int NS = D == 64 && QG == 1 ? 3 : 2;
   constexpr int kMaxGroup = 256;  // query heads per K/V head staged in LDS
   constexpr int KW_BYTES = 32 * RP;  // a wavefront's K rows
-  __shared__ __attribute__((aligned(1024))) char lds[NS * STAGE_BYTES];
+  __shared__ __attribute__((aligned(1024))) char lds_all[QG * NS * STAGE_BYTES];
   __shared__ __attribute__((aligned(1024))) char lds_k[kKLds ? NW * KW_BYTES : 16];
   __shared__ float head_c[2 * kMaxGroup];  // per query head of the group: c1, ALiBi slope
 
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave_wg = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = QG > 1 ? wave_wg / KW : 0;         // this wavefront's query group
+  const int wave = QG > 1 ? wave_wg % KW : wave_wg;  // and its index in the group
+  char* const lds = lds_all + grp * (NS * STAGE_BYTES);  // the group's stages
   const int lq = lane & 31, lh = lane >> 5;
 
   // workgroup -> (b, K/V head, residue, 128-key block); low blocks (seen by
@@ -538,7 +562,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(const BwdParams p
   MaskSpec ms = p.mask;
   ms.S = seq.len;
   const MaskGeom g = residue_geom(ms, r);
-  const int nblk_r = (g.S + 127) / 128;
+  const int nblk_r = (g.S + BK - 1) / BK;
   if (blk >= nblk_r) return;  // whole workgroup, before any barrier
   const int dil = p.mask.dil;
   const int64_t t0 = seq.tok0 + r;  // the residue's first token
@@ -550,7 +574,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(const BwdParams p
                 dkrs = p.dk_ss * dil, dvrs = p.dv_ss * dil;
 
   // the group's per-head score constants, once, before any DMA is in flight
-  for (int t = tid; t < p.G; t += NW * 64) {
+  for (int t = tid; t < p.G; t += NW * QG * 64) {
     const int hq = hkv * p.G + t;
     head_c[t] = p.scale * (p.head_scale ? p.head_scale[hq] : 1.0f);
     head_c[kMaxGroup + t] = (ALIBI && p.alibi_slopes) ? p.alibi_slopes[hq] * (float)p.mask.dil : 0.0f;
@@ -561,12 +585,15 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(const BwdParams p
   const float c1u = HEAD_C1 ? 1.0f : (D == 64 ? head_c[0] : uniform_f(head_c[0]));
 
   // this wavefront's 32 keys: K and V as MFMA B operands (lane = key); K rows
-  // kept in LDS are read by the wavefront that loads them, after its first wait
-  const int key0 = blk * 128 + 32 * wave;
+  // kept in LDS are loaded by group 0, which waits for them before the first
+  // step's barrier
+  const int key0 = blk * BK + 32 * wave;
   const int j = key0 + lq;
   const bool okj = j < g.S;
   bf16x8_t kf[kKLds ? 1 : DK], vf[DK];
-  if constexpr (kKLds) dma_rows<D, 1, 32>(kh, krs, imin32(key0, g.S - 1), g.S, lds_k + wave * KW_BYTES, 0, lane);
+  if constexpr (kKLds) {
+    if (grp == 0) dma_rows<D, 1, 32>(kh, krs, imin32(key0, g.S - 1), g.S, lds_k + wave * KW_BYTES, 0, lane);
+  }
   {
     const uint16_t* ks = kh + (int64_t)(okj ? j : 0) * krs + 8 * lh;
     const uint16_t* vs = vh + (int64_t)(okj ? j : 0) * vrs + 8 * lh;
@@ -578,9 +605,12 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(const BwdParams p
   }
 
   // query tiles of the rows that see the workgroup's keys, for each query head of the group
-  const RowSpan qs = query_range(g, blk * 128, imin32(blk * 128 + 127, g.S - 1));
-  const int t_lo = qs.lo / BM, n_qt = qs.lo <= qs.hi ? qs.hi / BM - t_lo + 1 : 0;
-  const int ntiles = n_qt * p.G;
+  const RowSpan qs = query_range(g, blk * BK, imin32(blk * BK + BK - 1, g.S - 1));
+  const int t_lo = qs.lo / BM, n_qt = qs.hi / BM - t_lo + 1;
+  // this group's tiles, and the steps of the group with the most (each passes
+  // a barrier in every wavefront of the workgroup)
+  const int ntiles = QG == 1 ? n_qt * p.G : (n_qt * p.G - grp + QG - 1) / QG;
+  const int nsteps = QG == 1 ? ntiles : (n_qt * p.G + QG - 1) / QG;
   const bool wvalid = key0 < g.S;
   const int kc = key0, kd = key0 + 31;
   // the rows that see this lane's key: an interval (exact for one key; empty
@@ -609,20 +639,29 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(const BwdParams p
     const uint16_t* dob;
     const float* sb;
   };
-  auto cursor0 = [&]() {
-    const int hq = hkv * p.G;
-    return Cursor{t_lo, hq, p.q + b * p.q_sb + hq * p.q_sh + t0 * p.q_ss,
-                  p.dout + b * p.do_sb + hq * p.do_sh + t0 * p.do_ss,
-                  p.stats + ((int64_t)(b * p.H + hq) * p.residues + r) * p.SR};
-  };
-  auto advance = [&](Cursor& c) {
-    if (++c.qt == t_lo + n_qt) {
-      c.qt = t_lo;
+  auto forward_by = [&](Cursor& c, int n) {  // n tiles on (n_qt >= 1: every row sees its own key)
+    c.qt += n;
+    auto next_head = [&]() {
+      c.qt -= n_qt;
       ++c.hq;
       c.qb += p.q_sh;
       c.dob += p.do_sh;
       c.sb += (int64_t)p.residues * p.SR;
+    };
+    if constexpr (QG == 1) {
+      if (c.qt == t_lo + n_qt) next_head();
+    } else {
+      while (c.qt >= t_lo + n_qt) next_head();
     }
+  };
+  auto advance = [&](Cursor& c) { forward_by(c, QG); };
+  auto cursor0 = [&]() {
+    const int hq = hkv * p.G;
+    Cursor c{t_lo, hq, p.q + b * p.q_sb + hq * p.q_sh + t0 * p.q_ss,
+             p.dout + b * p.do_sb + hq * p.do_sh + t0 * p.do_ss,
+             p.stats + ((int64_t)(b * p.H + hq) * p.residues + r) * p.SR};
+    if constexpr (QG > 1) forward_by(c, grp);
+    return c;
   };
   Cursor dc = cursor0(), cc = cursor0();
   // Scalar work per tile is kept small: the stage is a wrapping counter, the
@@ -637,10 +676,12 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(const BwdParams p
     qdma(dc.qb, qrs, i0, g.S, st, wave, lane);
     dodma(dc.dob, dors, i0, g.S, st + T_BYTES, wave, lane);
     if constexpr (kStats) {
-      // wavefront w moves BM / 2 floats: lse log2 e rows [w BM / 2, +BM / 2) (w < 2),
-      // or -delta rows [(w - 2) BM / 2, +BM / 2); the stats rows are padded to 64
-      const float* src = dc.sb + (wave >= 2 ? plane : 0) + i0 + BM / 2 * (wave & 1);
-      if (lane < BM / 2) dma4s(src, (uint32_t)(4 * lane), lds_addr(st + 2 * T_BYTES + 2 * BM * wave));
+      // the group's first KW / 2 wavefronts move lse log2 e, the others -delta,
+      // SN rows each; the stats rows are padded to 64
+      constexpr int SN = 2 * BM / KW;
+      static_assert((KW == 2 || KW == 4) && SN <= 64, "statistics per wavefront");
+      const float* src = dc.sb + (wave >= KW / 2 ? plane : 0) + i0 + SN * (wave & (KW / 2 - 1));
+      if (lane < SN) dma4s(src, (uint32_t)(4 * lane), lds_addr(st + 2 * T_BYTES + 4 * SN * wave));
     }
     advance(dc);
   };
@@ -655,7 +696,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(const BwdParams p
   }
 
   typedef short i16x8_t __attribute__((ext_vector_type(8)));
-  for (int it = 0; it < ntiles; ++it) {
+  for (int it = 0; it < nsteps; ++it) {
     if (dma_next - (it + 1) >= 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA2) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -666,6 +707,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(const BwdParams p
       issue(stage_behind<NS>(st_it));
       ++dma_next;
     }
+    if (QG > 1 && it >= ntiles) break;  // (the last step, in a group with one tile fewer)
     const char* St = lds + st_it * STAGE_BYTES;
     const int hq = cc.hq, i0 = cc.qt * BM;
     advance(cc);
@@ -742,6 +784,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(const BwdParams p
         pp[w] = pack_bf16x2(pv[2 * w], pv[2 * w + 1]);
         pd[w] = pack_bf16x2(dsv[2 * w], dsv[2 * w + 1]);
       }
+      // (the products' fragment reads stay below the scores: hoisted, they spill)
+      if constexpr (D == 128 && ALIBI && QG == 4 && NORM != NORM_RELU) __builtin_amdgcn_sched_barrier(0);
       // dV^T += dO^T P, dK^T += Q^T dS, 16-row chunk by chunk
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
@@ -764,6 +808,38 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(const BwdParams p
         }
       }
     }
+  }
+
+  if constexpr (QG > 1) {
+    // the groups' sums meet in LDS, dK and then dV: groups 1 .. QG - 1 write
+    // theirs lane-major over the stages, group 0 adds them in group order
+    constexpr int FL = 16 * DB * 64;  // floats of one wavefront's dK or dV
+    static_assert((QG - 1) * KW * FL * 4 <= (int)sizeof(lds_all), "the sums fit the stages");
+    float* const mb = reinterpret_cast<float*>(lds_all);
+    auto merge = [&](f32x16_t* acc) __attribute__((always_inline)) {
+      __syncthreads();  // every wavefront is past its last read of the stages
+      if (grp > 0) {
+        float* dst = mb + ((grp - 1) * KW + wave) * FL + lane;
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) dst[(16 * db + e) * 64] = acc[db][e];
+      }
+      __syncthreads();
+      if (grp == 0) {
+#pragma unroll
+        for (int q = 0; q < QG - 1; ++q) {
+          const float* src = mb + (q * KW + wave) * FL + lane;
+#pragma unroll
+          for (int db = 0; db < DB; ++db)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[db][e] += src[(16 * db + e) * 64];
+        }
+      }
+    };
+    merge(dk);
+    merge(dv);
+    if (grp > 0) return;
   }
 
   if (okj) {

@@ -120,6 +120,38 @@ def test_backward_d128_row_tile_edges(S, kw):
     _check(f"S={S} {kw}", grads, attention_grad_ref(q, k, v, do, **kw))
 
 
+# dK/dV workgroup shapes other than four key wavefronts in one group.  Few keys: two key
+# wavefronts and four query groups (lengths from one row tile, where groups stay empty, to
+# ragged tile counts; query heads of a K/V group that differ in scale).  256 workgroups of equal
+# walks: two query groups.
+SPLIT = [
+    *[(f"four_groups_S{S}_G{G}_d{D}", 1, 2 * G, 2, S, D, kw) for D in (64, 128) for G, kw in (
+        (1, dict(causal=True)), (3, dict(causal=True, head_scale=[0.5, 2.0, 1.0, 0.25, 1.5, 0.75])))
+      for S in (1, 33, 65, 130, 290)],
+    *[(f"two_groups_d{D}_{name}", 4, 16 * G, 16, 500, D, kw) for D in (64, 128) for G, name, kw in (
+        (1, "full", dict(causal=False)), (1, "sigmoid", dict(causal=False, norm="sigmoid", bias=-5.0)))],
+    ("two_groups_gqa_window_d64", 4, 32, 16, 500, 64, dict(causal=False, window=300)),
+]
+
+
+@pytest.mark.parametrize("name,B,H,Hkv,S,D,kw", SPLIT, ids=[e[0] for e in SPLIT])
+def test_backward_query_groups(name, B, H, Hkv, S, D, kw):
+    """dK/dV whose workgroups split the query tiles between groups and add the groups' sums;
+    the first and the last K/V head's query heads checked."""
+    _say(f"[bwd] split {name}")
+    q, k, v, do = _draw(B, H, Hkv, S, D, 4000 + S + D + H)
+    _, grads = _run(q, k, v, do, lambda a, b, c: attention(a, b, c, **kw))
+    G = H // Hkv
+    for b, hk in ((0, 0), (B - 1, Hkv - 1)):
+        hq = slice(hk * G, hk * G + G)
+        part = dict(kw)
+        if "head_scale" in kw:
+            part["head_scale"] = kw["head_scale"][hq]
+        refs = attention_grad_ref(q[b:b + 1, hq], k[b:b + 1, hk:hk + 1], v[b:b + 1, hk:hk + 1], do[b:b + 1, hq],
+                                  **part)
+        _check(f"{name} b={b} hk={hk}", [grads[0][b:b + 1, hq]] + [g[b:b + 1, hk:hk + 1] for g in grads[1:]], refs)
+
+
 def test_backward_causal_s2048_sampled_heads():
     """B2 H4 S2048 D64 causal softmax: the full kernel grid, two heads checked."""
     _say("[bwd] causal S2048")

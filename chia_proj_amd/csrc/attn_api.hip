@@ -275,8 +275,7 @@ int launch_fwd(const chia_attn_args* a, float* lse, void* stream) {
   if (geo.workgroups >= ((int64_t)1 << 31)) return CHIA_ATTN_ERR_SHAPE;
   p.n_wg = (int32_t)geo.workgroups;
   const int64_t slices = a->batch * a->heads * p.residues;
-  if (geo.rank && !a->cu_seqlens && slices % 8 == 0) p.rank_hx = (int32_t)(slices / 8);
-  p.div_hx = make_udiv(p.rank_hx > 0 ? p.rank_hx : 1);
+  p.order = launch_order(geo.rank, slices, a->heads, p.residues, a->cu_seqlens != nullptr);
   p.div_pairs = make_udiv(p.n_pairs);
   p.div_res = make_udiv(p.residues);
   p.div_h = make_udiv(p.H);
@@ -533,14 +532,12 @@ int launch_bwd(const chia_attn_bwd_args* ba, void* stream, bool noalloc) {
   // dQ first: with softmax it also writes the row statistics dK/dV reads.
   // Causal rows: each kernel launches its blocks with the most work first
   // (rank_order): the last query blocks (dQ), the first key blocks (dK/dV).
-  auto rank_for = [&](int64_t slices) {
-    const bool on = zigzag_of(p.mask) && !a->cu_seqlens && slices % 8 == 0;
-    p.rank_hx = on ? (int32_t)(slices / 8) : 0;
-    p.div_hx = make_udiv(on ? p.rank_hx : 1);
+  auto order_for = [&](int64_t heads) {
+    return launch_order(zigzag_of(p.mask), a->batch * heads * p.residues, heads, p.residues, a->cu_seqlens != nullptr);
   };
-  rank_for(a->batch * a->heads * p.residues);
+  p.order = order_for(a->heads);
   err = launch(ks.dq, g_dq, 256, p, s);
-  rank_for(a->batch * hkv * p.residues);
+  p.order = order_for(hkv);
   const int split = pick_dkdv_split(p.mask, a->batch * hkv * p.residues, G, a->head_dim == 64 ? 64 : 32);
   const DkdvSplit sp = kDkdvSplit[split];
   p.n_blk = (residue_geom(p.mask, 0).S + 32 * sp.kw - 1) / (32 * sp.kw);
@@ -589,12 +586,11 @@ extern "C" int chia_attn_fwd_fp8(const chia_attn_fp8_args* fa, void* stream) {
   p.n_blk = (residue_geom(p.mask, 0).S + 127) / 128;
   const int64_t bhr = a->batch * a->heads * p.residues;
   const int64_t n_wg = bhr * (int64_t)p.n_blk;
-  // Causal rows without a window: a block's work grows with its index, and the
-  // launch walks the longest blocks of every slice first (per XCD).
-  if (zigzag_of(p.mask) && !a->cu_seqlens && bhr % 8 == 0) p.rank_hx = (int32_t)(bhr / 8);
-  p.div_hx = make_udiv(p.rank_hx > 0 ? p.rank_hx : 1);
   if (n_wg >= ((int64_t)1 << 31)) return CHIA_ATTN_ERR_SHAPE;
   p.n_wg = (int32_t)n_wg;
+  // Causal rows without a window: a block's work grows with its index, and the
+  // launch walks the longest blocks of every slice first.
+  p.order = launch_order(zigzag_of(p.mask), bhr, a->heads, p.residues, a->cu_seqlens != nullptr);
   p.div_blk = make_udiv(p.n_blk);
   p.div_res = make_udiv(p.residues);
   p.div_h = make_udiv(p.H);

@@ -96,10 +96,7 @@ struct BwdParams {
   int32_t n_blk, n_wg;  // 128-row (or key) blocks per (b, head, residue 0); grid
   UDiv div_blk, div_res, div_h, div_g, div_hk, div_dil;
   float scale, softcap, bias, post_scale;
-  // Causal rows: the launched kernel's slices per XCD for the longest-first
-  // order (rank_order), 0 otherwise; and its divider.
-  int32_t rank_hx;
-  UDiv div_hx;
+  LaunchOrder order;  // the launched kernel's longest-first order (causal rows)
 };
 
 // Per-score gradient (see the header): from the raw s = q.k, dp = do.v and
@@ -309,8 +306,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(const BwdParams p) 
   // (packed sequences of unequal length: round-robin over the XCDs, no remap)
   // the query blocks with the most keys first
   int bhr, blk;
-  if (p.rank_hx > 0) {
-    const SliceUnit su = rank_order((int)blockIdx.x, p.rank_hx, p.div_hx, p.n_blk);
+  if (p.order.slices > 0) {
+    const SliceUnit su = rank_order((int)blockIdx.x, p.order, p.n_blk);
     bhr = su.slice;
     blk = su.unit;
   } else {
@@ -545,11 +542,12 @@ __global__ __launch_bounds__(64 * KW * QG, 2) void attn_bwd_dkdv_kernel(const Bw
   // the most rows under a causal mask) first
   const int HK = p.H / p.G;
   // the key blocks with the most queries (the first ones) first
-  int bhr, blk;
-  if (p.rank_hx > 0) {
-    const SliceUnit su = rank_order((int)blockIdx.x, p.rank_hx, p.div_hx, p.n_blk);
+  int bhr, blk = 0;
+  int unit = -1;  // longest-first: blocks counted from the sequence's last one
+  if (p.order.slices > 0) {
+    const SliceUnit su = rank_order((int)blockIdx.x, p.order, p.n_blk);
     bhr = su.slice;
-    blk = p.n_blk - 1 - su.unit;
+    unit = su.unit;
   } else {
     const int L = p.cu_seqlens ? (int)blockIdx.x : xcd_remap(blockIdx.x, p.n_wg);
     bhr = udiv(L, p.div_blk);
@@ -563,7 +561,8 @@ __global__ __launch_bounds__(64 * KW * QG, 2) void attn_bwd_dkdv_kernel(const Bw
   ms.S = seq.len;
   const MaskGeom g = residue_geom(ms, r);
   const int nblk_r = (g.S + BK - 1) / BK;
-  if (blk >= nblk_r) return;  // whole workgroup, before any barrier
+  if (unit >= 0) blk = nblk_r - 1 - unit;
+  if (blk < 0 || blk >= nblk_r) return;  // whole workgroup, before any barrier
   const int dil = p.mask.dil;
   const int64_t t0 = seq.tok0 + r;  // the residue's first token
   const uint16_t* kh = p.k + b * p.k_sb + hkv * p.k_sh + t0 * p.k_ss;

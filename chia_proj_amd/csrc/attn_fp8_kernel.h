@@ -68,10 +68,7 @@ struct Fp8Params {
   // seq_order[i] is the sequence of batch slot i (longest first).
   const int32_t* cu_seqlens;
   const int32_t* seq_order;
-  // Longest-first launch order for causal rows (fixed length, B H residues a
-  // multiple of 8): the (b, h, residue) slices per XCD, 0 otherwise; and its divider.
-  int32_t rank_hx;
-  UDiv div_hx;
+  LaunchOrder order;  // longest-first, for causal rows
 };
 
 // Swizzled 16-byte slot of chunk c of row r in an fp8 tile of D-byte rows.
@@ -124,15 +121,12 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_fp8_kernel(const Fp8Params p)
   const int lq = lane & 31, lh = lane >> 5;
 
   // workgroup -> (b, h, residue, 128-row block), the blocks with the most keys
-  // first.  Causal rows (rank_hx > 0): XCD x (workgroups x, x + 8, ...) serves
-  // slices [x rank_hx, (x + 1) rank_hx) and walks them rank by rank, every
-  // slice's last block, then every slice's second to last, ..., so the longest
-  // blocks all start first and the shortest fill the end of the launch.
-  // Otherwise each XCD gets a contiguous range of slices, longest block first
+  // first.  Causal rows: every slice's last block, then every slice's second
+  // to last, ... (LaunchOrder).  Otherwise each XCD gets a contiguous range of slices, longest block first
   // per slice; packed sequences go round-robin to the XCDs.
   int bhr, blk;
-  if (p.rank_hx > 0) {
-    const SliceUnit su = rank_order((int)blockIdx.x, p.rank_hx, p.div_hx, p.n_blk);
+  if (p.order.slices > 0) {
+    const SliceUnit su = rank_order((int)blockIdx.x, p.order, p.n_blk);
     bhr = su.slice;
     blk = su.unit;
   } else {

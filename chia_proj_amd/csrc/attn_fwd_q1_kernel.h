@@ -97,8 +97,8 @@ __global__ __launch_bounds__(256 * NG, Q1Config<D>::occupancy) void attn_fwd_q1_
 
   // ---- workgroup -> (batch, head, residue, unit) ----------------------------
   int bhr, pr;
-  if (p.rank_hx > 0) {
-    const SliceUnit su = rank_order((int)blockIdx.x, p.rank_hx, p.div_hx, p.n_pairs);
+  if (p.order.slices > 0) {
+    const SliceUnit su = rank_order((int)blockIdx.x, p.order, p.n_pairs);
     bhr = su.slice;
     pr = su.unit;
   } else {

@@ -139,6 +139,39 @@ def test_backward_each_sequence(name, lens, H, Hkv, D, kw):
             assert err.max().item() <= 1e-2 * m and err.mean().item() <= 1e-3 * m, (name, b, label)
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("H,Hkv", [(8, 8), (16, 8), (6, 3)])
+def test_causal_order_across_sequences(H, Hkv, D):
+    """Causal rows of unequal sequences, whose launches walk the blocks of every sequence
+    longest-first (heads per XCD when they divide by 8, round the XCDs otherwise): forward with a
+    prefix, and gradients, the first and last heads against the oracle."""
+    _say(f"[varlen] causal order H={H} Hkv={Hkv} D={D}")
+    lens, kw, G = [129, 700, 0, 1, 384], dict(causal=True), H // Hkv
+    q, k, v, cu = _packed(lens, H, Hkv, D, seed=60 + H + D)
+    do = torch.randn(q.shape, generator=torch.Generator().manual_seed(61)).to(torch.bfloat16)
+    qg, kg, vg = (t.to(DEV).requires_grad_(True) for t in (q, k, v))
+    attention_varlen(qg, kg, vg, cu.to(DEV), **kw).backward(do.to(DEV))
+    pre = attention_varlen(q.to(DEV), k.to(DEV), v.to(DEV), cu.to(DEV), prefix=100, **kw).cpu()
+    grads = [t.grad.cpu() for t in (qg, kg, vg)]
+    for b, L in enumerate(lens):
+        if L == 0:
+            continue
+        for hk in (0, Hkv - 1):
+            hq = slice(hk * G, hk * G + G)
+            part = [_seq(q, cu, b)[:, hq], *(_seq(t, cu, b)[:, hk:hk + 1] for t in (k, v))]
+            ref = attention_ref(*part, prefix=100, **kw)
+            for h in range(G):
+                res = gate.north_star_gate(ref[0, h], _seq(pre, cu, b)[0, hk * G + h].float())
+                assert res.ok, (b, hk, h, res.status, res.stats)
+            refs = attention_grad_ref(*part, _seq(do, cu, b)[:, hq], **kw)
+            floor = 1e-3 * max(r.abs().max().item() for r in refs)
+            got = [_seq(grads[0], cu, b)[:, hq], *(_seq(g, cu, b)[:, hk:hk + 1] for g in grads[1:])]
+            for label, g, r in zip(("dq", "dk", "dv"), got, refs):
+                m = max(r.abs().max().item(), floor, 1e-30)
+                err = (g.float() - r).abs()
+                assert err.max().item() <= 1e-2 * m and err.mean().item() <= 1e-3 * m, (b, hk, label)
+
+
 def test_backward_equal_lengths_bit_identical():
     _say("[varlen] backward equal lengths")
     B, S, H = 2, 400, 2

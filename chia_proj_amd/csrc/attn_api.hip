@@ -19,9 +19,9 @@ namespace chia {
 
 using KernelFn = void (*)(FwdParams);
 KernelFn select_kernel_d64(int waves, int norm, bool alibi, bool softcap);
-KernelFn select_q1_kernel_d64(int norm, bool alibi, bool softcap, bool cap_fixed);
+KernelFn select_q1_kernel_d64(int which, bool alibi, bool softcap, bool cap_fixed);
 KernelFn select_kernel_d128(int norm);
-KernelFn select_q1_kernel_d128(int norm, bool alibi, bool softcap, bool cap_fixed);
+KernelFn select_q1_kernel_d128(int which, bool alibi, bool softcap, bool cap_fixed);
 KernelFn select_q1_split_kernel_d128(int norm, bool alibi, bool softcap, bool cap_fixed);
 BwdKernels select_bwd_kernels_d64(int norm, bool alibi, bool softcap);
 BwdKernels select_bwd_kernels_d128(int norm, bool alibi, bool softcap);
@@ -98,7 +98,7 @@ ScorePath score_path_of(const chia_attn_args* a) {
   return sp;
 }
 
-// Launch geometry shared by chia_attn_fwd and the planner.
+// Launch geometry of chia_attn_fwd; the planner's nominal schedule.
 struct Geometry {
   int waves;       // wavefronts per workgroup
   int rows;        // rows per row block (32 per wavefront)
@@ -107,8 +107,8 @@ struct Geometry {
   int residues;
   int zigzag;
   bool q1;         // the one-block core (attn_fwd_q1_kernel.h)
-  int groups;      // one-block core: groups of `waves` wavefronts per workgroup (2: a
-                   // zigzag pair's steps split between two groups)
+  int shape;       // one-block core: the workgroup's shape (Q1Shape)
+  int groups;      // and its groups of `waves` wavefronts
   bool rank;       // launch the units with the most keys first (rank_order)
   int64_t workgroups;
 };
@@ -119,6 +119,7 @@ Geometry paired_geometry(const MaskSpec& m, int64_t batch, int64_t heads) {
   geo.residues = num_residues(m);
   geo.zigzag = zigzag_of(m) ? 1 : 0;
   geo.q1 = false;
+  geo.shape = Q1_ONE;
   geo.groups = 1;
   geo.rank = false;
   const int32_t s0 = residue_geom(m, 0).S;  // longest residue class
@@ -139,7 +140,8 @@ Geometry paired_geometry(const MaskSpec& m, int64_t batch, int64_t heads) {
   return geo;
 }
 
-// The forward's core and geometry.  Head dim 64: the paired core, or for a
+// The nominal schedule, which chia_attn_plan describes and launch_geometry
+// starts from.  Head dim 64: the paired core, or for a
 // window or block mask, causal rows with a prefix, and causal softmax on the
 // grids named below, the one-block core at four wavefronts per SIMD (north
 // star: local 53.2 -> 42.6 us, sliding window 53.1 -> 42.9, block-diagonal
@@ -154,7 +156,7 @@ Geometry paired_geometry(const MaskSpec& m, int64_t batch, int64_t heads) {
 // rows runs the one-block core: the paired softmax kernel at head_dim 128
 // spills (17 VGPRs at one wavefront per SIMD), and the one-block core
 // measured 288.8 against 294.7 us (B4 H16 S4096, temperature).
-Geometry forward_geometry(const chia_attn_args* a, const MaskSpec& m, const ScorePath& sp) {
+Geometry plan_geometry(const chia_attn_args* a, const MaskSpec& m, const ScorePath& sp) {
   Geometry geo = paired_geometry(m, a->batch, a->heads);
   const bool banded = m.hi < kInf || m.blk > 0;
   const int32_t s0 = residue_geom(m, 0).S;
@@ -205,7 +207,124 @@ Geometry forward_geometry(const chia_attn_args* a, const MaskSpec& m, const Scor
   // Head dim 128, zigzag pairs on fewer than two workgroups per CU: one group
   // per workgroup would leave one wavefront per SIMD, so two groups split
   // each pair's steps (every SIMD then holds two wavefronts).
-  if (a->head_dim == 128 && geo.zigzag && geo.workgroups < 2 * kCUs) geo.groups = 2;
+  if (a->head_dim == 128 && geo.zigzag && geo.workgroups < 2 * kCUs) {
+    geo.shape = Q1_ZIGZAG2;
+    geo.groups = 2;
+  }
+  return geo;
+}
+
+// The geometry a forward is launched with.  plan_geometry's schedule is one of
+// the candidates; the others are the one-block core's shapes (Q1Shape) with the
+// blocks longest-first on causal rows, whose key groups serve grids too small
+// to fill the chip or bound by their longest block: one 128-row block by two
+// groups (KEYS2), 64 rows by four (KEYS4).  The candidate with the least
+// estimated time is taken.  The unit is one (128 rows x 64 keys) step on a
+// fully occupied CU; n workgroups with walks of at most `longest` and on
+// average `mean` steps take at least
+//   * the steps of all spread evenly, and
+//   * k (P_k) for the k-th round of CUs, P_k the length of walk 256 (k - 1) in
+//     falling order (taken as falling linearly), times what the k resident
+//     workgroups lose to a CU with fewer wavefronts than it could hold
+//     (head_dim 64: 2.2 with 4 of 16, 1.05 with 8; head_dim 128: 1.3 with 4 of 8),
+// times the shape's cost per step, plus its start-up (and merge) per round.
+// The paired core (full rows) and the zigzag pairs (causal rows, head_dim 128)
+// have equal walks and run in whole rounds of two workgroups per CU (one, with
+// two groups per pair).  The constants fit 690 timed shapes (1-4 sequences of
+// 128-8192 tokens, 4-32 heads, every mask and normaliser): 0.6 % above the best
+// candidate on average, and 1.37x (head_dim 64) and 1.22x (128) faster than
+// plan_geometry's schedule on drawn shapes, at most 3 % slower but for one 11 us
+// call.  For instance B1 H12 S3000 D64 causal: pairs 63 us, one block per
+// workgroup 49, KEYS2 37, KEYS4 28; B1 H32/16 S2500 D128 softcap 107, 77, 85,
+// 107; B4 H16 S2048 D64 causal 49, 48, 53, 63.
+struct StepCost {
+  double per_step[4], start[4];  // by Q1Shape
+  double paired[3], zigzag, zigzag2;
+};
+constexpr StepCost kCostD64 = {{1.0, 0.0, 1.35, 1.75}, {1.6, 0.0, 4.7, 6.6}, {0.93, 0.88, 0.88}, 0.0, 0.0};
+constexpr StepCost kCostD128 = {{1.0, 0.0, 1.1, 1.6}, {4.0, 0.0, 5.0, 6.0}, {1.0, 0.8, 0.85}, 0.99, 1.09};
+
+// Rounds of equal walks of `w` steps, two workgroups per CU; the last round's
+// workgroups run alone on their CUs when it has at most one per CU.
+double equal_rounds(double n, double w, double alone) {
+  const double full = std::ceil(n / (2 * kCUs)) - 1.0;
+  return w * (2.0 * full + (n - 2.0 * kCUs * full > kCUs ? 2.0 : alone));
+}
+
+Geometry launch_geometry(const chia_attn_args* a, const MaskSpec& m, const ScorePath& sp) {
+  Geometry geo = plan_geometry(a, m, sp);
+  const bool d64 = a->head_dim == 64;
+  const bool banded = m.hi < kInf || m.blk > 0, causal = zigzag_of(m), softmax = a->norm == CHIA_ATTN_NORM_SOFTMAX;
+  const MaskGeom g = residue_geom(m, 0);
+  const int32_t nblk = (g.S + 127) / 128;
+  // Packed sequences: the launch is sized for the longest one and their lengths
+  // are not known here; the others are taken to add up to what makes 0.4 (0.5)
+  // of the grid real, and banded masks keep one block per workgroup.
+  const bool packed = a->cu_seqlens != nullptr;
+  const double slices = (double)(a->batch * a->heads * geo.residues) * (!packed ? 1.0 : d64 ? 0.4 : 0.5);
+  // Causal softmax at head_dim 64 whose pairs are exactly one round of two
+  // workgroups per CU, of whole tiles: every CU ends at the same time and the
+  // pairs stay (B1 H16 S8192: 154.7 against 163.3 us, ALiBi 154 against 163;
+  // B2 H16 S4096 85.7 against 86.5).
+  if (d64 && !packed && geo.zigzag && !geo.q1 && geo.waves == 4 && geo.workgroups == 2 * kCUs && softmax &&
+      !sp.softcap && g.S % 256 == 0)
+    return geo;
+  // key tiles of the first, the middle and the last block
+  auto walk = [&](int32_t blk) {
+    const TileRange t = tile_range(g, blk * 128, imin32(blk * 128 + 127, g.S - 1), kBN);
+    return (double)(t.n_pre + t.n2);
+  };
+  const double w0 = walk(0), w1 = walk(nblk / 2), w2 = walk(nblk - 1);
+  const double longest = std::fmax(w0, std::fmax(w1, w2)), mean = 0.25 * (w0 + 2.0 * w1 + w2);
+
+  const StepCost& sc = d64 ? kCostD64 : kCostD128;
+  auto shape_cost = [&](int shape) {
+    const double unit = shape == Q1_KEYS4 ? 0.5 : 1.0, n = slices * nblk / unit;
+    const int waves = shape == Q1_ONE ? 4 : 8, most = d64 ? 16 : 8;
+    const double fall = 2.0 * (longest - mean) * kCUs / n;
+    double t = n * mean * unit / kCUs;
+    for (int k = 1; k <= 8 && (k == 1 || (k - 1) * kCUs < n); ++k) {
+      const int w = k * waves;
+      const double loss = w >= most ? 1.0 : !d64 ? 1.3 : w == 4 ? 2.2 : w == 8 ? 1.05 : 1.025;
+      const double len = longest - fall * (k - 1);
+      t = t > k * len * unit * loss ? t : k * len * unit * loss;
+    }
+    // softcap at head_dim 64: KEYS4's short steps hide its longer score chain
+    const double cap = !(d64 && sp.softcap) ? 1.0 : shape == Q1_KEYS2 ? 1.2 : shape == Q1_KEYS4 ? 0.8 : 1.0;
+    return sc.per_step[shape] * cap * t + sc.start[shape] * std::fmax(1.0, n * waves / (kCUs * most));
+  };
+  int shape = Q1_ONE;
+  double best = shape_cost(Q1_ONE);
+  bool keep = false;  // plan_geometry's paired or zigzag schedule
+  const double n_pair = slices * ((nblk + 1) / 2);
+  if (!geo.q1 && !causal && geo.waves == 4) {
+    const double t = sc.paired[a->norm] * std::fmax(2.0 * longest * n_pair / kCUs, equal_rounds(n_pair, 2.0 * longest, 1.3));
+    keep = !packed && t + sc.start[Q1_ONE] < best;
+    if (keep) best = t + sc.start[Q1_ONE];
+  } else if (!d64 && geo.zigzag) {
+    const double w = 2.0 * mean;
+    const double t = n_pair >= 2 * kCUs ? sc.zigzag * std::fmax(w * n_pair / kCUs, equal_rounds(n_pair, w, 1.3))
+                                        : sc.zigzag2 * std::ceil(n_pair / kCUs) * w;
+    keep = t + sc.start[Q1_ONE] < best;
+    if (keep) best = t + sc.start[Q1_ONE];
+  }
+  if (!(packed && banded))
+    for (int s : {Q1_KEYS2, Q1_KEYS4})
+      if (const double t = shape_cost(s); t < (banded ? 0.85 : 1.0) * best) {
+        shape = s;
+        best = t;
+        keep = false;
+      }
+  if (keep) return geo;
+  geo.q1 = true;
+  geo.zigzag = 0;
+  geo.rank = causal;
+  geo.shape = shape;
+  geo.waves = shape == Q1_KEYS4 ? 2 : 4;
+  geo.groups = shape == Q1_ONE ? 1 : shape == Q1_KEYS2 ? 2 : 4;
+  geo.rows = 32 * geo.waves;
+  geo.n_pairs = (g.S + geo.rows - 1) / geo.rows;
+  geo.workgroups = a->batch * a->heads * geo.residues * geo.n_pairs;
   return geo;
 }
 
@@ -267,7 +386,7 @@ int launch_fwd(const chia_attn_args* a, float* lse, void* stream) {
   p.lse_sh = a->cu_seqlens ? 1 : a->seqlen;
   p.lse_ss = a->cu_seqlens ? a->heads : 1;
   const ScorePath sp = score_path_of(a);
-  const Geometry geo = forward_geometry(a, p.mask, sp);
+  const Geometry geo = launch_geometry(a, p.mask, sp);
   p.residues = geo.residues;
   p.n_pairs = geo.n_pairs;
   p.zigzag = geo.zigzag;
@@ -291,11 +410,14 @@ int launch_fwd(const chia_attn_args* a, float* lse, void* stream) {
   // (attn_fwd_q1_kernel.h); north star 208.7 -> 200.6 us, headline 66.7 ->
   // 62.7 us against the running max.
   const bool cap_fixed = sp.softcap && a->norm == CHIA_ATTN_NORM_SOFTMAX && a->softcap * kLog2e <= 78.0f;
-  KernelFn fn = a->head_dim == 64 ? (geo.q1 ? select_q1_kernel_d64((int)a->norm, sp.alibi, sp.softcap, cap_fixed)
-                                            : select_kernel_d64(waves, (int)a->norm, sp.alibi, sp.softcap))
-               : geo.q1            ? (geo.groups == 2 ? select_q1_split_kernel_d128((int)a->norm, sp.alibi, sp.softcap, cap_fixed)
-                                                  : select_q1_kernel_d128((int)a->norm, sp.alibi, sp.softcap, cap_fixed))
-                                   : select_kernel_d128((int)a->norm);
+  const int norm = (int)a->norm, which = norm + kNorms * geo.shape;
+  KernelFn fn;
+  if (!geo.q1)
+    fn = a->head_dim == 64 ? select_kernel_d64(waves, norm, sp.alibi, sp.softcap) : select_kernel_d128(norm);
+  else if (geo.shape == Q1_ZIGZAG2)
+    fn = select_q1_split_kernel_d128(norm, sp.alibi, sp.softcap, cap_fixed);
+  else
+    fn = (a->head_dim == 64 ? select_q1_kernel_d64 : select_q1_kernel_d128)(which, sp.alibi, sp.softcap, cap_fixed);
   if (fn == nullptr) return CHIA_ATTN_ERR_NORM;  // no instantiation for this core and normaliser
   void* kargs[] = {&p};
   hipError_t err = hipLaunchKernel(reinterpret_cast<const void*>(fn), dim3((unsigned)p.n_wg),
@@ -617,7 +739,7 @@ extern "C" int chia_attn_plan(const chia_attn_args* a, chia_attn_plan_info* out)
   if (!out) return CHIA_ATTN_ERR_NULL;
   std::memset(out, 0, sizeof(*out));
   const MaskSpec spec = spec_of(a);
-  const Geometry geo = forward_geometry(a, spec, score_path_of(a));
+  const Geometry geo = plan_geometry(a, spec, score_path_of(a));
   const int bn = kBN;
   const int64_t bhn = a->batch * a->heads;
   // The paired core computes two row blocks per KV tile in 32 x 64 sub-tiles;

@@ -8,23 +8,36 @@ namespace chia {
 
 using KernelFn = void (*)(FwdParams);
 
-template <int NORM, bool AL, bool SC, bool CAPFIX = false>
+template <int NORM, bool AL, bool SC, int NG, int RW, int KG, bool CAPFIX = false>
 static KernelFn inst_q1() {
-  return attn_fwd_q1_kernel<64, NORM, AL, SC, 1, CAPFIX>;
+  return attn_fwd_q1_kernel<64, NORM, AL, SC, NG, CAPFIX, RW, KG>;
 }
 
-KernelFn select_q1_kernel_d64(int norm, bool alibi, bool softcap, bool cap_fixed) {
+template <int NG, int RW, int KG>
+static KernelFn select_shape(int norm, bool alibi, bool softcap, bool cap_fixed) {
   if (cap_fixed && norm == NORM_SOFTMAX && softcap)
-    return alibi ? inst_q1<NORM_SOFTMAX, true, true, true>() : inst_q1<NORM_SOFTMAX, false, true, true>();
+    return alibi ? inst_q1<NORM_SOFTMAX, true, true, NG, RW, KG, true>()
+                 : inst_q1<NORM_SOFTMAX, false, true, NG, RW, KG, true>();
   static const KernelFn table[3][2][2] = {
-      {{inst_q1<NORM_SOFTMAX, false, false>(), inst_q1<NORM_SOFTMAX, false, true>()},
-       {inst_q1<NORM_SOFTMAX, true, false>(), inst_q1<NORM_SOFTMAX, true, true>()}},
-      {{inst_q1<NORM_SIGMOID, false, false>(), inst_q1<NORM_SIGMOID, false, true>()},
-       {inst_q1<NORM_SIGMOID, true, false>(), inst_q1<NORM_SIGMOID, true, true>()}},
-      {{inst_q1<NORM_RELU, false, false>(), inst_q1<NORM_RELU, false, true>()},
-       {inst_q1<NORM_RELU, true, false>(), inst_q1<NORM_RELU, true, true>()}},
+      {{inst_q1<NORM_SOFTMAX, false, false, NG, RW, KG>(), inst_q1<NORM_SOFTMAX, false, true, NG, RW, KG>()},
+       {inst_q1<NORM_SOFTMAX, true, false, NG, RW, KG>(), inst_q1<NORM_SOFTMAX, true, true, NG, RW, KG>()}},
+      {{inst_q1<NORM_SIGMOID, false, false, NG, RW, KG>(), inst_q1<NORM_SIGMOID, false, true, NG, RW, KG>()},
+       {inst_q1<NORM_SIGMOID, true, false, NG, RW, KG>(), inst_q1<NORM_SIGMOID, true, true, NG, RW, KG>()}},
+      {{inst_q1<NORM_RELU, false, false, NG, RW, KG>(), inst_q1<NORM_RELU, false, true, NG, RW, KG>()},
+       {inst_q1<NORM_RELU, true, false, NG, RW, KG>(), inst_q1<NORM_RELU, true, true, NG, RW, KG>()}},
   };
   return table[norm][alibi ? 1 : 0][softcap ? 1 : 0];
+}
+
+// `which`: normaliser + kNorms times the shape (Q1Shape).
+KernelFn select_q1_kernel_d64(int which, bool alibi, bool softcap, bool cap_fixed) {
+  const int norm = which % kNorms;
+  switch (which / kNorms) {
+    case Q1_ONE: return select_shape<1, 4, 1>(norm, alibi, softcap, cap_fixed);
+    case Q1_KEYS2: return select_shape<1, 4, 2>(norm, alibi, softcap, cap_fixed);
+    case Q1_KEYS4: return select_shape<1, 2, 4>(norm, alibi, softcap, cap_fixed);
+  }
+  return nullptr;
 }
 
 }  // namespace chia

@@ -1,7 +1,7 @@
 // attn_fwd_q1_kernel.h -- the one-block forward core: one 32-row query block
-// per wavefront.  It runs every head_dim 128 forward but long full rows of
-// sigmoid / ReLU, and at head_dim 64 the banded masks (window, block), causal
-// rows with a prefix, and causal softmax on large grids.
+// per wavefront.  It runs every forward but long full rows on grids of whole
+// rounds of the paired core's workgroups (and causal softmax at head_dim 64
+// on exactly one such round).
 //
 // Reference semantics: the eager closures of extra_bench.py:32-62 and
 // sigmoid_fix.py:34-40, as for attn_fwd_kernel.h, whose helpers (DMA, LDS
@@ -27,7 +27,17 @@
 //   * a workgroup of 4 wavefronts owns row blocks of 128 rows of one (batch,
 //     head, dilation residue); each wavefront owns 32 of them (one query
 //     block, ONE MFMA stream);
-//   * for a causal band without a window (zigzag), a workgroup processes
+//   * key groups (KG > 1): small grids leave CUs idle or end with the longest
+//     block's walk, one dependent step after another on a nearly empty CU
+//     (about 1.15 us per 64 keys at head_dim 64 against 0.59 us of a full CU's
+//     time).  KG groups of RW wavefronts then share a block of 32 RW rows: key
+//     tile s belongs to group s % KG, each group has its own LDS stages, O, m
+//     and l, and the partial results meet in LDS at the end with the
+//     log-sum-exp rescale.  {4, 2}: 128 rows, two groups; {2, 4}: 64 rows, four
+//     groups (32-key tiles, so that their stages fit).  B1 H8 S512 D64 softcap
+//     16.6 -> 9.9 us, B1 H12 S3000 D64 causal 63.5 -> 28.1 us (the launch rule
+//     and its figures: attn_api.hip, launch_geometry);
+//   * on zigzag launches (causal rows, head_dim 128) a workgroup processes
 //     block i and then block n-1-i, one after the other, so every workgroup
 //     does the same work; otherwise one block;
 //   * the K / V tiles (64 keys) of the block's key range go HBM -> LDS with
@@ -44,9 +54,9 @@
 
 namespace chia {
 
-// Waves per SIMD the register budget targets, and LDS stages per workgroup:
-// head_dim 64, four workgroups per CU x 2 stages x 16 KB; head_dim 128, two
-// workgroups per CU x 2 stages x 32 KB.
+// Waves per SIMD the register budget targets, and LDS stages per group:
+// head_dim 64, four workgroups of one group per CU x 2 stages x 16 KB;
+// head_dim 128, two x 2 stages x 32 KB.
 template <int D>
 struct Q1Config {
   static_assert(D == 64 || D == 128, "head_dim 64 or 128");
@@ -58,12 +68,13 @@ struct Q1Config {
 // zigzag pair's steps between them (below); NG = 1: one group.  CAPFIX
 // (softcap softmax with cap log2 e <= 78, chosen by the host): the weights are
 // taken against a fixed reference (below) instead of a running max.
-template <int D, int NORM, bool ALIBI, bool SOFTCAP, int NG = 1, bool CAPFIX = false>
-__global__ __launch_bounds__(256 * NG, Q1Config<D>::occupancy) void attn_fwd_q1_kernel(const FwdParams p) {
+template <int D, int NORM, bool ALIBI, bool SOFTCAP, int NG = 1, bool CAPFIX = false, int RW = 4, int KG = 1>
+__global__ __launch_bounds__(64 * RW * NG * KG, Q1Config<D>::occupancy) void attn_fwd_q1_kernel(const FwdParams p) {
   static_assert(NG == 1 || NG == 2, "one or two groups");
+  static_assert(KG == 1 || NG == 1, "a zigzag pair's groups, or key groups");
   static_assert(!CAPFIX || (SOFTCAP && NORM == NORM_SOFTMAX), "the fixed reference is for softcap softmax");
-  constexpr int NW = 4;  // wavefronts per group
-  constexpr int BN = kBN;
+  constexpr int NW = RW;  // wavefronts per group
+  constexpr int BN = KG == 4 ? 32 : kBN;  // keys per tile (four groups' stages in the LDS)
   constexpr int NT = NW * 64;
   constexpr int BM = NW * 32;          // rows per block
   constexpr int DK = D / 16;           // k-steps of the QK^T MFMA
@@ -85,13 +96,13 @@ __global__ __launch_bounds__(256 * NG, Q1Config<D>::occupancy) void attn_fwd_q1_
   constexpr bool kRawRelu = (NORM == NORM_RELU) && !ALIBI && !SOFTCAP;
   constexpr bool kCapR = SOFTCAP && NORM == NORM_SOFTMAX;
   constexpr bool kSigFold = NORM == NORM_SIGMOID && !ALIBI && !SOFTCAP;
-  __shared__ __attribute__((aligned(1024))) char lds_all[NG * NS * STAGE_BYTES];
+  __shared__ __attribute__((aligned(1024))) char lds_all[NG * KG * NS * STAGE_BYTES];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave_wg = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int grp = NG == 2 ? wave_wg >> 2 : 0;  // this wavefront's group
-  const int wave = wave_wg & (NW - 1);          // and its index in the group
+  const int grp = NG * KG > 1 ? wave_wg / NW : 0;  // this wavefront's group
+  const int wave = wave_wg & (NW - 1);             // and its index in the group
   char* const lds = lds_all + grp * (NS * STAGE_BYTES);  // the group's LDS stages
   const int lq = lane & 31, lh = lane >> 5;
 
@@ -117,7 +128,7 @@ __global__ __launch_bounds__(256 * NG, Q1Config<D>::occupancy) void attn_fwd_q1_
   const MaskGeom g = residue_geom(ms, r);
   const int nblk = (g.S + BM - 1) / BM;
   int blk0, blk1;
-  if (p.zigzag) {
+  if (KG == 1 && p.zigzag) {
     blk0 = pr;
     blk1 = nblk - 1 - pr;
     if (blk1 < blk0) return;  // whole workgroup, before any barrier
@@ -218,10 +229,13 @@ __global__ __launch_bounds__(256 * NG, Q1Config<D>::occupancy) void attn_fwd_q1_
   // (O, m, l).  Each group streams its own tiles through its own LDS stages;
   // the workgroup barrier of every step is shared, so both groups pass the same
   // number of barriers: the group with fewer steps adds empty ones.
+  // KG > 1 (key groups): one block; step s belongs to group s % KG, whose own
+  // steps are numbered 0, 1, ...  The merge at the end is the same.
   int M = NG == 2 ? (nsteps + 1) / 2 : nsteps;
   if (NG == 2 && blk1 >= 0 && M < n0) M = n0;  // (not reached for causal pairs)
-  const int s_lo = grp == 1 ? M : 0, s_hi = grp == 1 ? nsteps : M;
-  const int n_bar = imax32(M, nsteps - M);  // step barriers of each group
+  const int s_lo = KG == 1 && grp == 1 ? M : 0;
+  const int s_hi = KG > 1 ? (nsteps - grp + KG - 1) / KG : grp == 1 ? nsteps : M;
+  const int n_bar = KG > 1 ? (nsteps + KG - 1) / KG : imax32(M, nsteps - M);  // step barriers of each group
   // pass (0: block 0, 1: block 1) that both groups compute part of, or -1
   const int split_pass =
       NG == 2 && M > 0 && M < nsteps ? (blk1 >= 0 ? (M > n0 ? 1 : -1) : 0) : -1;
@@ -282,7 +296,7 @@ __global__ __launch_bounds__(256 * NG, Q1Config<D>::occupancy) void attn_fwd_q1_
   int dma_next = s_lo;
   int jt_dma = 0, brk = 0;
   for (; dma_next < s_lo + NS - 1 && dma_next < s_hi; ++dma_next) {
-    jt_dma = step_key0(dma_next);
+    jt_dma = step_key0(KG > 1 ? grp + dma_next * KG : dma_next);
     brk = next_break(dma_next);
     issue_step(dma_next, jt_dma);
   }
@@ -307,13 +321,13 @@ __global__ __launch_bounds__(256 * NG, Q1Config<D>::occupancy) void attn_fwd_q1_
   int step = s_lo;
   bool merged = false;
 #pragma unroll 1
-  for (int pass = 0; pass < 2; ++pass) {
+  for (int pass = 0; pass < (KG > 1 ? 1 : 2); ++pass) {
     const int blk = pass == 0 ? blk0 : blk1;
     if (blk < 0) break;
     const int nt = pass == 0 ? n0 : tr1.n_pre + tr1.n2;
     // this group's steps of the block: [it_lo, it_hi)
     const int base = pass == 0 ? 0 : n0;
-    const int it_lo = imax32(s_lo - base, 0), it_hi = imin32(s_hi - base, nt);
+    const int it_lo = imax32(s_lo - base, 0), it_hi = KG > 1 ? n_bar : imin32(s_hi - base, nt);
     if (it_lo >= it_hi) continue;
     const int row0 = blk * BM + 32 * wave;
     const bool valid = row0 < g.S;
@@ -355,9 +369,12 @@ __global__ __launch_bounds__(256 * NG, Q1Config<D>::occupancy) void attn_fwd_q1_
       }
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
+      if (KG > 1 && it >= s_hi) break;  // (the last step, in a group with one step fewer)
       const int jt0 = jt_dma;  // this step's first key
       if (dma_next < s_hi) {
-        if (dma_next == brk) {
+        if constexpr (KG > 1) {
+          jt_dma = step_key0(grp + dma_next * KG);
+        } else if (dma_next == brk) {
           jt_dma = step_key0(dma_next);
           brk = next_break(dma_next);
         } else {
@@ -369,8 +386,8 @@ __global__ __launch_bounds__(256 * NG, Q1Config<D>::occupancy) void attn_fwd_q1_
       const char* St = lds + ((uint32_t)step & (NS - 1)) * STAGE_BYTES;
 
 #pragma unroll
-      for (int kbs = 0; kbs < 2; ++kbs) {
-        const int kb = kRev ? 1 - kbs : kbs;
+      for (int kbs = 0; kbs < BN / 32; ++kbs) {
+        const int kb = kRev ? BN / 32 - 1 - kbs : kbs;
         const int jb = jt0 + 32 * kb;
         const int cls = key_class(kr, jb);
         if (cls == TILE_EMPTY) continue;
@@ -557,45 +574,53 @@ __global__ __launch_bounds__(256 * NG, Q1Config<D>::occupancy) void attn_fwd_q1_
       }
     }
 
-    // ---- the block both groups computed part of: merge through LDS -------------
-    if constexpr (NG == 2) {
-      if (pass == split_pass) {
+    // ---- the block several groups computed part of: merge through LDS ----------
+    if constexpr (NG * KG > 1) {
+      if (KG > 1 || pass == split_pass) {
         merged = true;
-        for (int k = s_hi - s_lo; k < n_bar; ++k) __builtin_amdgcn_s_barrier();
+        if constexpr (KG == 1)
+          for (int k = s_hi - s_lo; k < n_bar; ++k) __builtin_amdgcn_s_barrier();
         // every wavefront is past its last step (no DMA in flight, no stage
-        // still read): the stages of both groups hold the merge buffer, per
-        // wavefront of group 1 its 16 DB accumulators, m and l, lane-major
+        // still read): the stages hold the merge buffer, per wavefront of the
+        // groups after the first its 16 DB accumulators, m and l, lane-major
         constexpr int FL = 16 * DB + 2;
-        float* mb = reinterpret_cast<float*>(lds_all) + wave * (FL * 64) + lane;
+        static_assert((NG * KG - 1) * NW * FL * 64 * 4 <= (int)sizeof(lds_all), "the partial results fit the stages");
+        float* const mb = reinterpret_cast<float*>(lds_all) + lane;
         __syncthreads();
-        if (grp == 1) {
+        if (grp > 0) {
+          float* dst = mb + ((grp - 1) * NW + wave) * (FL * 64);
 #pragma unroll
           for (int db = 0; db < DB; ++db)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) mb[(16 * db + e) * 64] = oacc[db][e];
-          mb[(16 * DB) * 64] = m_run;
-          mb[(16 * DB + 1) * 64] = l_run;
+            for (int e = 0; e < 16; ++e) dst[(16 * db + e) * 64] = oacc[db][e];
+          dst[(16 * DB) * 64] = m_run;
+          dst[(16 * DB + 1) * 64] = l_run;
         }
         __syncthreads();
-        if (grp == 1) return;  // group 0 stores the block
-        const float m1 = mb[(16 * DB) * 64], l1 = mb[(16 * DB + 1) * 64];
-        if constexpr (NORM == NORM_SOFTMAX) {
-          // both partials against the larger reference (a row neither group
-          // saw keeps m = -inf, O = 0 and l = 0)
-          const float mm = fmaxf(m_run, m1);
-          const float a0 = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - mm);
-          const float a1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - mm);
+        if (grp > 0) return;  // group 0 stores the block
+#pragma unroll 1
+        for (int q = 0; q < NG * KG - 1; ++q) {
+          const float* src = mb + (q * NW + wave) * (FL * 64);
+          const float m1 = src[(16 * DB) * 64], l1 = src[(16 * DB + 1) * 64];
+          if constexpr (NORM == NORM_SOFTMAX) {
+            // both partials against the larger reference (a row neither group
+            // saw keeps m = -inf, O = 0 and l = 0)
+            const float mm = fmaxf(m_run, m1);
+            const float a0 = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - mm);
+            const float a1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - mm);
 #pragma unroll
-          for (int db = 0; db < DB; ++db)
+            for (int db = 0; db < DB; ++db)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) oacc[db][e] = __builtin_fmaf(oacc[db][e], a0, mb[(16 * db + e) * 64] * a1);
-          l_run = __builtin_fmaf(l_run, a0, l1 * a1);
-          m_run = mm;
-        } else {
+              for (int e = 0; e < 16; ++e)
+                oacc[db][e] = __builtin_fmaf(oacc[db][e], a0, src[(16 * db + e) * 64] * a1);
+            l_run = __builtin_fmaf(l_run, a0, l1 * a1);
+            m_run = mm;
+          } else {
 #pragma unroll
-          for (int db = 0; db < DB; ++db)
+            for (int db = 0; db < DB; ++db)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) oacc[db][e] += mb[(16 * db + e) * 64];
+              for (int e = 0; e < 16; ++e) oacc[db][e] += src[(16 * db + e) * 64];
+          }
         }
       }
     }

@@ -219,7 +219,9 @@ typedef struct chia_attn_fp8_args {
 
 int chia_attn_fwd_fp8(const chia_attn_fp8_args* args, void* stream);
 
-/* Host-only schedule statistics for `args` (no GPU call).  Used by the
+/* Host-only statistics of the nominal schedule for `args` (no GPU call): the
+ * launch may take another core or split the blocks' keys between groups of
+ * wavefronts where the grid is small, over the same tiles.  Used by the
  * benchmark's FLOP accounting; the reference has no counterpart (its timer,
  * extra_bench.py:8-22, counts latency only). */
 typedef struct chia_attn_plan_info {

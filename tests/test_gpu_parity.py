@@ -418,3 +418,35 @@ def test_grouped_query_kv(name, H, Hkv, S, D, kw):
     r = oracle.attention_ref(q, k, v, **kw)
     res = gate.north_star_gate(r, o.float().cpu(), scale_aware=kw.get("norm", "softmax") != "softmax")
     assert res.ok, f"{name}: {res.status} {res.stats}"
+
+
+# Forwards whose workgroups split a block's keys between groups of wavefronts: small grids (64 rows
+# by four groups) from one row to ragged tile counts, where groups stay without a tile, and 192
+# blocks of full rows (128 rows by two groups).
+KEY_GROUPS = [
+    *[(f"four_groups_S{S}_d{D}_{n}", 1, 2, S, D, kw) for D in (64, 128) for S in (1, 33, 65, 127, 129, 300, 511)
+      for n, kw in (("causal", dict(causal=True)), ("full_relu", dict(causal=False, norm="relu", post_scale=0.01)))],
+    *[(f"four_groups_{n}_d{D}", 1, 3, 450, D, kw) for D in (64, 128) for n, kw in (
+        ("softcap", dict(causal=True, softcap=30.0)), ("softcap80", dict(causal=True, softcap=80.0)),
+        ("alibi", dict(causal=True, alibi_slopes=[0.5, 0.1, -0.05])), ("prefix", dict(causal=True, prefix=100)),
+        ("sigmoid", dict(causal=False, norm="sigmoid", bias=-6.0)), ("window", dict(causal=True, window=200)),
+        ("dilation", dict(causal=True, dilation=2)))],
+    *[(f"two_groups_{n}_d{D}", 2, 12, 1001, D, kw) for D in (64, 128) for n, kw in (
+        ("full", dict(causal=False)), ("alibi", dict(causal=False, alibi_slopes=[0.01 * h for h in range(12)])),
+        ("sigmoid", dict(causal=False, norm="sigmoid", bias=-6.0)))],
+]
+
+
+@pytest.mark.parametrize("name,B,H,S,D,kw", KEY_GROUPS, ids=[c[0] for c in KEY_GROUPS])
+def test_key_groups(name, B, H, S, D, kw):
+    _say(f"[parity] key groups {name}")
+    g = torch.Generator("cpu").manual_seed(S + D + H)
+    q, k, v = (torch.randn(B, H, S, D, generator=g).to(torch.bfloat16) for _ in range(3))
+    o = attention(q.to(DEV), k.to(DEV), v.to(DEV), **kw).float().cpu()
+    for b, h in {(0, 0), (B - 1, H - 1)}:
+        part = dict(kw)
+        if "alibi_slopes" in kw:
+            part["alibi_slopes"] = kw["alibi_slopes"][h:h + 1]
+        ref = oracle.attention_ref(*(t[b:b + 1, h:h + 1] for t in (q, k, v)), **part)
+        res = gate.north_star_gate(ref, o[b:b + 1, h:h + 1], scale_aware=kw.get("norm", "softmax") != "softmax")
+        assert res.ok, (name, b, h, res.status, res.stats)

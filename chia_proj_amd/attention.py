@@ -10,6 +10,7 @@ leaves synchronisation to the caller, extra_bench.py:12,19).
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import math
 import threading
@@ -17,9 +18,11 @@ import weakref
 from collections import OrderedDict
 from typing import Optional, Sequence, Union
 
+import numpy as np
 import torch
 
 from . import _lib
+from .library import eager_fwd, eager_fwd_varlen, plain_eager
 
 PerHead = Union[None, torch.Tensor, Sequence[float]]
 
@@ -76,6 +79,10 @@ def _per_head_vector(vals: PerHead, heads: int, device: torch.device, name: str,
         if t.device != device:
             raise ValueError(f"{name} is on {t.device}, tensors are on {device}")
         return t.to(torch.float32).contiguous()
+    if cache and type(vals) is tuple and len(vals) == heads:  # e.g. the variants' presets: seen before
+        cached = _vec_cache.get((name, device.index, vals))
+        if cached is not None:
+            return cached
     # host values: checked in Python (no tensor op, so fake-tensor tracing can run this)
     if isinstance(vals, torch.Tensor):
         if not cache:  # tracing: the values are not read on the host (nor checked)
@@ -160,9 +167,12 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, norm: str = 
                   post_scale=post_scale)
     needs_grad = torch.is_grad_enabled() and any(isinstance(t, torch.Tensor) and t.requires_grad for t in (q, k, v))
     if needs_grad or torch.compiler.is_compiling():
-        # the registered operator: autograd (chia_attn::bwd) and torch.compile see one node
+        # the registered operator: autograd (chia_attn::bwd) and torch.compile see one
+        # node; plain eager tensors: the same implementation without its dispatch
         if out is not None:
             raise ValueError("out= is not supported when q, k or v requires grad or under torch.compile")
+        if not torch.compiler.is_compiling() and plain_eager(q, k, v) and q.dim() == 4:
+            return eager_fwd(q, k, v, _device_params(params, q))
         return _op_forward(q, k, v, params)[0]
     # Fast path: a call with the same shapes, layouts and parameters as an
     # earlier one reuses its validated argument struct and per-head vectors;
@@ -274,6 +284,79 @@ def _strides3(t: torch.Tensor):
     return t.stride(0), t.stride(1), t.stride(2)
 
 
+def _device_params(params, q):
+    """`params` with the per-head values as float32 vectors on q's device (q: [.., H, ..]
+    at dim 1, on the GPU, not traced)."""
+    p = dict(params)
+    if p["head_scale"] is not None:
+        p["head_scale"] = _per_head_vector(p["head_scale"], q.shape[1], q.device, "head_scale", positive=True)
+    if p["alibi_slopes"] is not None:
+        p["alibi_slopes"] = _per_head_vector(p["alibi_slopes"], q.shape[1], q.device, "alibi_slopes", positive=False)
+    return p
+
+
+def run_forward(q, k, v, params):
+    """(o, lse) by chia_attn_fwd_lse: o contiguous, lse float32 [B, H, S] (softmax) or [0]."""
+    softmax = params["norm"] == "softmax"
+    hs_in, sl_in = params["head_scale"], params["alibi_slopes"]
+    key = _training_key("fwd", (q, k, v), params)
+    cache = _args_cache()
+    a = cache.get(key) if key is not None else None
+    if a is not None:
+        ptrs = (q.data_ptr(), k.data_ptr(), v.data_ptr())
+        if not (ptrs[0] | ptrs[1] | ptrs[2]) & 15:
+            o = torch.empty(q.shape, dtype=torch.bfloat16, device=q.device)
+            lse = torch.empty(q.shape[:3] if softmax else (0,), dtype=torch.float32, device=q.device)
+            a.q, a.k, a.v, a.o = *ptrs, o.data_ptr()
+            a.head_scale = hs_in.data_ptr() if hs_in is not None else None
+            a.alibi_slopes = sl_in.data_ptr() if sl_in is not None else None
+            with _device_of(q):
+                _lib.fwd_lse(a, lse.data_ptr() if softmax else 0, _current_stream(q))
+            return o, lse
+    o = torch.empty(q.shape, dtype=torch.bfloat16, device=q.device)  # contiguous, as the operator's fake
+    # Every tensor _prepare returns (layout copies of q, k, v and the per-head
+    # vectors) stays referenced until the launch is queued: a copy freed earlier
+    # would hand its memory to lse while the struct still points at it.
+    a, hs, sl, qkv, _o = _prepare(q, k, v, o, **params)
+    lse = torch.empty(q.shape[:3] if softmax else (0,), dtype=torch.float32, device=q.device)
+    with torch.cuda.device(q.device):
+        _lib.fwd_lse(a, lse.data_ptr() if softmax else 0, torch.cuda.current_stream(q.device).cuda_stream)
+    if key is not None and qkv[0] is q and qkv[1] is k and qkv[2] is v:
+        cache[key] = a
+        if len(cache) > _ARGS_CACHE_MAX:
+            cache.popitem(last=False)
+    del qkv, hs, sl  # queued: torch's allocator orders any reuse after the launch on this stream
+    return o, lse
+
+
+_NO_SWITCH = contextlib.nullcontext()
+
+
+def _device_of(t):
+    """Context with t's device current (no switch, and none of its cost, when it already is)."""
+    return _NO_SWITCH if torch.cuda.current_device() == t.get_device() else torch.cuda.device(t.device)
+
+
+def _training_key(tag, tensors, params):
+    """Key of a validated argument struct: the tensors' shapes, types, layouts and
+    devices and every parameter; None when the full path has to look at the call
+    (per-head vectors it would convert, unhashable values)."""
+    try:
+        vecs = (params["head_scale"], params["alibi_slopes"])
+        for t in vecs:
+            if t is not None and not (isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == torch.float32
+                                      and t.is_contiguous()):
+                return None
+        key = (tag, params["norm"], params["causal"], params["window"], params["dilation"], params["block"],
+               params["prefix"], params["scale"], params["softcap"], params["bias"], params["post_scale"],
+               tuple(None if t is None else (t.shape, t.device) for t in vecs),
+               tuple((t.shape, t.dtype, t.device, t.stride()) for t in tensors))
+        hash(key)
+        return key
+    except (AttributeError, TypeError):
+        return None
+
+
 def _op_forward(q, k, v, params):
     """(o, lse) through torch.ops.chia_attn.fwd, per-head values as float32 device vectors."""
     from .library import call_fwd
@@ -297,18 +380,7 @@ def run_backward(do, q, k, v, o, lse, params):
     # of an earlier one (per-head values arrive as float32 device vectors) reuses
     # its validated argument structs; only the data pointers are new.
     hs_in, sl_in = params["head_scale"], params["alibi_slopes"]
-    try:
-        key = ("bwd", q.shape, q.dtype, q.device, q.stride(), k.shape, k.dtype, k.stride(), v.shape, v.dtype,
-               v.stride(), o.shape, o.dtype, o.stride(), do.shape, do.dtype, do.stride(), lse is None,
-               params["norm"], params["causal"], params["window"], params["dilation"], params["block"],
-               params["prefix"], params["scale"], params["softcap"], params["bias"], params["post_scale"],
-               tuple(None if t is None else (tuple(t.shape), t.device) for t in (hs_in, sl_in)))
-        # device vectors the full path would pass through unchanged (float32, contiguous)
-        if not all(t is None or (isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == torch.float32
-                                 and t.is_contiguous()) for t in (hs_in, sl_in)):
-            key = None
-    except (AttributeError, TypeError):
-        key = None
+    key = _training_key("bwd" if lse is None else "bwd_lse", (q, k, v, o, do), params)
     cache = _args_cache()
     entry = cache.get(key) if key is not None else None
     if entry is not None:
@@ -568,13 +640,23 @@ def check_cu_seqlens(cu_seqlens, total: int, max_seqlen: Optional[int] = None) -
     cu[0] = 0, non-decreasing, cu[B] = total tokens.  Returns (B, max length)
     (max_seqlen if given, which must be >= every length).  Reads the values on the
     host (a device tensor is copied back: one synchronisation)."""
+    _check_cu_tensor(cu_seqlens)
+    host, lens, longest = _host_cu_seqlens(cu_seqlens, total, max_seqlen)
+    return len(lens), longest
+
+
+def _check_cu_tensor(cu_seqlens) -> None:
     if not isinstance(cu_seqlens, torch.Tensor) or cu_seqlens.dim() != 1 or cu_seqlens.numel() < 2:
         raise ValueError("cu_seqlens must be a 1-D tensor of batch + 1 token offsets")
     if cu_seqlens.dtype.is_floating_point or cu_seqlens.dtype == torch.bool:
         raise TypeError(f"cu_seqlens must be an integer tensor, got {cu_seqlens.dtype}")
-    host = cu_seqlens.detach().to("cpu", torch.int64)
+
+
+def _host_cu_seqlens(cu_seqlens, total: int, max_seqlen: Optional[int]):
+    """(offsets, lengths, longest) of checked offsets, as numpy int64 arrays."""
+    host = cu_seqlens.detach().to("cpu", torch.int64).numpy()
     lens = host[1:] - host[:-1]
-    if int(host[0]) != 0 or bool((lens < 0).any()) or int(host[-1]) != total:
+    if int(host[0]) != 0 or int(lens.min()) < 0 or int(host[-1]) != total:
         raise ValueError(f"cu_seqlens must start at 0, be non-decreasing and end at the {total} packed tokens")
     if total >= (1 << 31):
         raise ValueError("at most 2^31 - 1 packed tokens")
@@ -583,7 +665,7 @@ def check_cu_seqlens(cu_seqlens, total: int, max_seqlen: Optional[int] = None) -
         if int(max_seqlen) < longest:
             raise ValueError(f"max_seqlen {max_seqlen} is shorter than the longest sequence ({longest})")
         longest = int(max_seqlen)
-    return int(lens.numel()), longest
+    return host, lens, longest
 
 
 _CU_CACHE_MAX = 32
@@ -605,11 +687,11 @@ def _cu_plan(cu_seqlens, total: int, max_seqlen: Optional[int], device):
         if hit is not None and hit[0]() is cu_seqlens:
             _cu_cache.move_to_end(key)
             return hit[1]
-    B, S = check_cu_seqlens(cu_seqlens, total, max_seqlen)
-    host = cu_seqlens.detach().to("cpu", torch.int64)
-    order = torch.argsort(host[1:] - host[:-1], descending=True, stable=True).to(torch.int32).to(device)
-    cu = host.to(torch.int32).to(device)
-    out = (B, S, cu, order)
+    _check_cu_tensor(cu_seqlens)
+    host, lens, longest = _host_cu_seqlens(cu_seqlens, total, max_seqlen)
+    order = np.argsort(-lens, kind="stable")
+    both = torch.from_numpy(np.concatenate((host, order)).astype(np.int32)).to(device)  # one copy
+    out = (len(lens), longest, both[:len(host)], both[len(host):])
     if key is not None:
         _cu_cache[key] = (weakref.ref(cu_seqlens), out)
         if len(_cu_cache) > _CU_CACHE_MAX:
@@ -681,6 +763,9 @@ def attention_varlen(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_seqle
     if needs_grad or torch.compiler.is_compiling():
         if out is not None:
             raise ValueError("out= is not supported when q, k or v requires grad or under torch.compile")
+        if (not torch.compiler.is_compiling() and plain_eager(q, k, v) and q.dim() == 3
+                and type(cu_seqlens) is torch.Tensor and cu_seqlens.is_cuda):
+            return eager_fwd_varlen(q, k, v, cu_seqlens, max_seqlen, _device_params(params, q))
         return _op_forward_varlen(q, k, v, cu_seqlens, max_seqlen, params)[0]
     if isinstance(q, torch.Tensor) and q.dim() == 3 and q.shape[0] == 0:
         check_cu_seqlens(cu_seqlens, 0, max_seqlen)

@@ -25,7 +25,6 @@ from typing import Optional, Tuple
 import torch
 from torch import Tensor
 
-from . import _lib
 
 NAMESPACE = "chia_attn"
 
@@ -41,24 +40,10 @@ def _params(norm, causal, window, dilation, block, prefix, scale, head_scale, al
 def fwd(q: Tensor, k: Tensor, v: Tensor, norm: str, causal: bool, window: int, dilation: int, block: int,
         prefix: int, scale: Optional[float], head_scale: Optional[Tensor], alibi_slopes: Optional[Tensor],
         softcap: float, bias: float, post_scale: float) -> Tuple[Tensor, Tensor]:
-    from .attention import _prepare
+    from .attention import run_forward
 
-    p = _params(norm, causal, window, dilation, block, prefix, scale, head_scale, alibi_slopes, softcap, bias,
-                post_scale)
-    o = torch.empty(q.shape, dtype=torch.bfloat16, device=q.device)  # contiguous, as the fake
-    # Every tensor _prepare returns (layout copies of q, k, v and the per-head
-    # vectors) stays referenced until the launch is queued: a copy freed earlier
-    # would hand its memory to lse while the struct still points at it.
-    a, hs, sl, qkv, _o = _prepare(q, k, v, o, **p)
-    B, H, S, _ = q.shape
-    if norm == "softmax":
-        lse = torch.empty(B, H, S, dtype=torch.float32, device=q.device)
-    else:
-        lse = torch.empty(0, dtype=torch.float32, device=q.device)
-    with torch.cuda.device(q.device):
-        _lib.fwd_lse(a, lse.data_ptr() if lse.numel() else 0, torch.cuda.current_stream(q.device).cuda_stream)
-    del qkv, hs, sl  # queued: torch's allocator orders any reuse after the launch on this stream
-    return o, lse
+    return run_forward(q, k, v, _params(norm, causal, window, dilation, block, prefix, scale, head_scale,
+                                        alibi_slopes, softcap, bias, post_scale))
 
 
 @fwd.register_fake
@@ -99,16 +84,19 @@ def _setup_context(ctx, inputs, output):
     ctx.set_materialize_grads(False)  # no zero-filled gradient for the unused lse
 
 
+def _traced(do: Tensor) -> bool:
+    """torch.compile, make_fx / AOTAutograd (a dispatch mode is active), or fake / meta
+    tensors: the backward is the registered operator, one node of the graph.  Eager on
+    the GPU it is the same implementation without a second operator dispatch."""
+    return (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0
+            or type(do) is not torch.Tensor or do.device.type != "cuda")
+
+
 def _backward(ctx, do, _dlse):
     q, k, v, o, lse = ctx.saved_tensors
     if do is None:
         return (None,) * (3 + len(ctx.rest))
-    # traced (torch.compile, make_fx / AOTAutograd: a dispatch mode is active, or
-    # fake / meta tensors): the registered operator, one node of the graph;
-    # eager on the GPU: the same implementation without a second operator dispatch
-    traced = (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0
-              or type(do) is not torch.Tensor or do.device.type != "cuda")
-    if traced:
+    if _traced(do):
         dq, dk, dv = torch.ops.chia_attn.bwd(do, q, k, v, o, lse, *ctx.rest)
     else:
         from .attention import run_backward
@@ -120,15 +108,63 @@ def _backward(ctx, do, _dlse):
 fwd.register_autograd(_backward, setup_context=_setup_context)
 
 
-def call_fwd(q: Tensor, k: Tensor, v: Tensor, params: dict) -> Tuple[Tensor, Tensor]:
-    """torch.ops.chia_attn.fwd with attention()'s keyword parameters (per-head
+def _schema_args(params: dict) -> tuple:
+    """attention()'s keyword parameters as the operators' trailing arguments (per-head
     vectors already float32 device tensors or None; scale None = default)."""
-    return torch.ops.chia_attn.fwd(q, k, v, params["norm"], bool(params["causal"]), int(params["window"] or 0),
-                                   int(params["dilation"] or 1), int(params["block"] or 0),
-                                   int(params["prefix"] or 0),
-                                   None if params["scale"] is None else float(params["scale"]),
-                                   params["head_scale"], params["alibi_slopes"], float(params["softcap"] or 0.0),
-                                   float(params["bias"]), float(params["post_scale"]))
+    return (params["norm"], bool(params["causal"]), int(params["window"] or 0), int(params["dilation"] or 1),
+            int(params["block"] or 0), int(params["prefix"] or 0),
+            None if params["scale"] is None else float(params["scale"]), params["head_scale"],
+            params["alibi_slopes"], float(params["softcap"] or 0.0), float(params["bias"]),
+            float(params["post_scale"]))
+
+
+def call_fwd(q: Tensor, k: Tensor, v: Tensor, params: dict) -> Tuple[Tensor, Tensor]:
+    """torch.ops.chia_attn.fwd with attention()'s keyword parameters."""
+    return torch.ops.chia_attn.fwd(q, k, v, *_schema_args(params))
+
+
+# ---- eager training ------------------------------------------------------------------
+# The operators' dispatch (schema parsing, the autograd wrapper's pytree maps, one
+# Python call per dispatch key) costs more host time than the rest of an eager
+# training call together.  Plain CUDA tensors outside every mechanism that needs to
+# see the operator take the same implementations through an autograd function of
+# their own, which saves the tensors the registered formula saves.
+
+_PLAIN_TYPES = (Tensor, torch.nn.Parameter)
+
+
+def plain_eager(*tensors) -> bool:
+    """True when nothing can observe whether the operator itself was dispatched: plain
+    CUDA tensors, no dispatch or function mode (tracing, FakeTensor, profiling
+    modes), no functorch transform (vmap, grad, jvp), no forward-mode level and no
+    TorchScript tracing."""
+    for t in tensors:
+        if type(t) not in _PLAIN_TYPES or not t.is_cuda:
+            return False
+    return (torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
+            and not torch._C._are_functorch_transforms_active()
+            and torch.autograd.forward_ad._current_level < 0 and torch._C._get_tracing_state() is None)
+
+
+class _EagerAttention(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, q, k, v, *rest):
+        from .attention import run_forward
+
+        o, lse = run_forward(q, k, v, _params(*rest))
+        ctx.rest = rest
+        ctx.save_for_backward(q, k, v, o, lse)
+        ctx.set_materialize_grads(False)
+        return o
+
+    @staticmethod
+    def backward(ctx, do):
+        return _backward(ctx, do, None)
+
+
+def eager_fwd(q: Tensor, k: Tensor, v: Tensor, params: dict) -> Tensor:
+    """call_fwd()'s o, differentiable, for plain_eager() tensors."""
+    return _EagerAttention.apply(q, k, v, *_schema_args(params))
 
 
 # ---- packed variable-length batches ------------------------------------------------
@@ -195,7 +231,13 @@ def _backward_varlen(ctx, do, _dlse):
     q, k, v, o, lse, cu_seqlens = ctx.saved_tensors
     if do is None:
         return (None,) * (4 + len(ctx.rest))
-    dq, dk, dv = torch.ops.chia_attn.bwd_varlen(do, q, k, v, o, lse, cu_seqlens, *ctx.rest)
+    if _traced(do):
+        dq, dk, dv = torch.ops.chia_attn.bwd_varlen(do, q, k, v, o, lse, cu_seqlens, *ctx.rest)
+    else:
+        from .attention import run_backward_varlen
+
+        max_seqlen, *rest = ctx.rest
+        dq, dk, dv = run_backward_varlen(do, q, k, v, o, lse, cu_seqlens, _max_len(max_seqlen), _params(*rest))
     return (dq, dk, dv) + (None,) * (1 + len(ctx.rest))
 
 
@@ -205,14 +247,29 @@ fwd_varlen.register_autograd(_backward_varlen, setup_context=_setup_context_varl
 def call_fwd_varlen(q: Tensor, k: Tensor, v: Tensor, cu_seqlens: Tensor, max_seqlen: Optional[int],
                     params: dict) -> Tuple[Tensor, Tensor]:
     """torch.ops.chia_attn.fwd_varlen with attention_varlen()'s keyword parameters."""
-    return torch.ops.chia_attn.fwd_varlen(q, k, v, cu_seqlens, int(max_seqlen or 0), params["norm"],
-                                          bool(params["causal"]), int(params["window"] or 0),
-                                          int(params["dilation"] or 1), int(params["block"] or 0),
-                                          int(params["prefix"] or 0),
-                                          None if params["scale"] is None else float(params["scale"]),
-                                          params["head_scale"], params["alibi_slopes"],
-                                          float(params["softcap"] or 0.0), float(params["bias"]),
-                                          float(params["post_scale"]))
+    return torch.ops.chia_attn.fwd_varlen(q, k, v, cu_seqlens, int(max_seqlen or 0), *_schema_args(params))
+
+
+class _EagerAttentionVarlen(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, q, k, v, cu_seqlens, max_seqlen, *rest):
+        from .attention import run_forward_varlen
+
+        o, lse = run_forward_varlen(q, k, v, cu_seqlens, _max_len(max_seqlen), _params(*rest))
+        ctx.rest = (max_seqlen, *rest)
+        ctx.save_for_backward(q, k, v, o, lse, cu_seqlens)
+        ctx.set_materialize_grads(False)
+        return o
+
+    @staticmethod
+    def backward(ctx, do):
+        return _backward_varlen(ctx, do, None)
+
+
+def eager_fwd_varlen(q: Tensor, k: Tensor, v: Tensor, cu_seqlens: Tensor, max_seqlen: Optional[int],
+                     params: dict) -> Tensor:
+    """call_fwd_varlen()'s o, differentiable, for plain_eager() tensors."""
+    return _EagerAttentionVarlen.apply(q, k, v, cu_seqlens, int(max_seqlen or 0), *_schema_args(params))
 
 
 # ---- FP8 forward -----------------------------------------------------------------

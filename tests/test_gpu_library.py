@@ -6,6 +6,7 @@ import math
 
 import pytest
 import torch
+import torch.utils.checkpoint
 
 import chia_proj_amd  # noqa: F401
 from chia_proj_amd import attention, gate
@@ -201,3 +202,83 @@ def test_layout_copies_live_through_the_launch(norm):
             m = max(rr.abs().max().item(), floor)
             err = (got - rr).abs()
             assert err.max().item() <= 1e-2 * m and err.mean().item() <= 1e-3 * m, (b, label)
+
+
+EAGER_KW = [dict(causal=True, window=70), dict(norm="sigmoid", causal=False, bias=-2.0),
+            dict(causal=True, head_scale=[0.5, 1.0, 2.0, 1.5])]
+
+
+@pytest.mark.parametrize("kw", EAGER_KW, ids=["window", "sigmoid", "head_scale"])
+@pytest.mark.parametrize("packed", [False, True])
+def test_eager_training_matches_the_operator(kw, packed):
+    """Plain eager tensors skip the operator's dispatch: outputs and gradients are the
+    operator's bit for bit, under saved-tensor hooks and checkpointing too, and the tensors
+    offered to the hooks are the same."""
+    from chia_proj_amd import attention_varlen
+    from chia_proj_amd.attention import _op_forward, _op_forward_varlen
+
+    _say(f"[lib] eager training {kw} packed={packed}")
+    cu = torch.tensor([0, 130, 300], dtype=torch.int32, device=DEV)
+    full = dict(norm="softmax", causal=True, window=0, dilation=1, block=0, prefix=0, scale=None, head_scale=None,
+                alibi_slopes=None, softcap=0.0, bias=0.0, post_scale=1.0)
+    full.update(kw)
+    q, k, v = _qkv(1, 4, 2, 300, 64, seed=8)
+    if packed:
+        q, k, v = (t[0].transpose(0, 1).contiguous() for t in (q, k, v))
+    do = torch.randn(q.shape, generator=torch.Generator("cpu").manual_seed(9)).to(torch.bfloat16).to(DEV)
+
+    def eager(a, b, c):
+        return attention_varlen(a, b, c, cu, 170, **kw) if packed else attention(a, b, c, **kw)
+
+    def operator(a, b, c):
+        return (_op_forward_varlen(a, b, c, cu, 170, full) if packed else _op_forward(a, b, c, full))[0]
+
+    def grads(fn, hooks=False):
+        seen = []
+        ts = [t.clone().requires_grad_(True) for t in (q, k, v)]
+        if hooks:
+            with torch.autograd.graph.saved_tensors_hooks(lambda t: (seen.append(tuple(t.shape)), t.cpu())[1],
+                                                          lambda t: t.to(DEV)):
+                o = fn(*ts)
+        else:
+            o = fn(*ts)
+        return [o, *torch.autograd.grad(o, ts, do)], seen
+
+    want, want_seen = grads(operator, hooks=True)
+    for fn, hooks in ((eager, False), (eager, True),
+                      (lambda *t: torch.utils.checkpoint.checkpoint(eager, *t, use_reentrant=False), False)):
+        got, seen = grads(fn, hooks)
+        for a, b in zip(got, want):
+            assert torch.equal(a, b)
+        if hooks:
+            assert seen == want_seen
+
+
+def test_eager_training_leaves_transforms_to_the_operator():
+    """Function modes, dispatch modes and functorch transforms still meet the operator."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from chia_proj_amd.library import plain_eager
+
+    q, k, v = _qkv(1, 2, 2, 64, 64, seed=3, grad=True)
+    assert plain_eager(q, k, v) and not plain_eager(q.cpu(), k, v)
+
+    class Fn(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Dispatch(TorchDispatchMode):
+        names = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.names.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    with Fn():
+        assert not plain_eager(q, k, v)
+    with Dispatch() as mode:
+        attention(q, k, v)
+    assert any("chia_attn.fwd" in n for n in mode.names)
+    with pytest.raises(RuntimeError):  # torch.func.grad through a custom operator: refused by torch
+        torch.func.grad(lambda a: attention(a, k.detach(), v.detach()).float().sum())(q.detach())

@@ -437,7 +437,7 @@ extern "C" int chia_attn_fwd_lse(const chia_attn_args* a, float* lse, void* stre
 
 namespace {
 constexpr int kBwdMaxGroup = 256;  // query heads per K/V head the dK/dV kernel stages
-constexpr int kBwdBlock = 128;     // rows per dQ workgroup (dK/dV: 32 keys per key wavefront)
+constexpr int kBwdBlock = 128;     // rows (dQ) or keys (dK/dV) of a block by four wavefronts
 
 // Rows of the stats workspace per (b, h, residue): residue 0's length padded
 // to the 64-row tiles the dK/dV kernel reads whole.
@@ -449,54 +449,74 @@ int64_t bwd_workspace(const chia_attn_args* a) {
   return 2 * a->batch * a->heads * (int64_t)num_residues(m) * stats_rows(m) * (int64_t)sizeof(float);
 }
 
-// Which workgroup shape the dK/dV kernel takes (kDkdvSplit), by an estimate of
-// the launch's time on 256 CUs.  The unit is one (128-key, row tile) step on a
-// fully occupied CU.  A launch of n workgroups of KW key wavefronts and QG
-// groups, whose walks have the longest length `l`, is bound by
+// Which workgroup shape (kBwdSplit) a backward kernel takes, by an estimate of
+// the launch's time on 256 CUs.  The unit is one (128 rows or keys, tile) step on
+// a fully occupied CU.  A launch of n workgroups of `own` wavefronts' rows and
+// `groups` groups, whose walks have at most `longest` steps and `mean` on
+// average, is bound by
 //   * the work of all of them spread evenly, or
 //   * the k-th round of CUs: k (P_k) where P_k is about the length of walk
 //     number 256 (k - 1) in falling order (the lengths taken as falling
 //     linearly from the longest), a workgroup of four wavefronts that is alone
-//     on its CU running at 1 / 1.3 of the CU's rate,
-// times what the split costs per step (1.05 for two groups: one workgroup per
-// CU instead of two, so start and end overlap less; 1.6 for four: each Q / dO
-// tile serves 64 keys instead of 128), plus 4 steps per round of start-up and
-// 2 more for adding the groups' sums.  The constants fit 110 drawn shapes (1-4
-// sequences of 128-4096 tokens, 1-32 K/V heads, every mask): within 0.3 % of
-// the best shape on average, never more than 3 % above {4, 1}, which by itself
-// was 21 % above the best (up to 1.9x: B1 H32/8 S3000 D128 causal, dQ + dK/dV
-// 561 us against 424 {4, 2} and 305 {2, 4}; B4 H16 S4096 D64 490 against 567
-// and 657).
-int pick_dkdv_split(const MaskSpec& m, int64_t slices, int64_t group, int32_t row_tile) {
-  const MaskGeom g = residue_geom(m, 0);
-  const int32_t nblk = (g.S + kBwdBlock - 1) / kBwdBlock;
-  // walks of the first, the middle and the last key block
-  auto walk = [&](int32_t blk) {
-    const RowSpan r = query_range(g, blk * kBwdBlock, imin32(blk * kBwdBlock + kBwdBlock - 1, g.S - 1));
-    return (double)group * (r.hi / row_tile - r.lo / row_tile + 1);
-  };
-  const double w0 = walk(0), w1 = walk(nblk / 2), w2 = walk(nblk - 1);
-  const double longest = std::fmax(w0, std::fmax(w1, w2)), mean = 0.25 * (w0 + 2.0 * w1 + w2);
-  constexpr double kPerStep[kDkdvSplits] = {1.0, 1.05, 1.6};
+//     on its CU running at 1 / `alone` of the CU's rate,
+// times what the split costs per step (two groups: one workgroup per CU instead
+// of two, so start and end overlap less; four: each tile serves 64 rows or keys
+// instead of 128, in 32-key steps for dQ), plus start-up and merge per round.
+struct SplitCost {
+  double alone, per_step[kBwdSplits], start[kBwdSplits];
+};
+// dK/dV: fit on 110 drawn shapes (1-4 sequences of 128-4096 tokens, 1-32 K/V
+// heads, every mask): within 0.3 % of the best shape on average, never more
+// than 3 % above {4, 1}, which by itself was 21 % above the best (up to 1.9x:
+// B1 H32/8 S3000 D128 causal, dQ + dK/dV 561 us against 424 {4, 2} and 305
+// {2, 4}; B4 H16 S4096 D64 490 against 567 and 657).
+constexpr SplitCost kDkdvCost = {1.3, {1.0, 1.05, 1.6}, {4.0, 6.0, 6.0}};
+// dQ: fit on 200 drawn shapes, 0.1-0.2 % above the best; {4, 1} by itself 3 %
+// (dQ + dK/dV, up to 1.28x at head_dim 64 and 1.23x at 128).
+constexpr SplitCost kDqCostD64 = {1.5, {1.0, 0.95, 1.3}, {3.6, 7.0, 6.7}};
+constexpr SplitCost kDqCostD128 = {1.45, {1.0, 1.13, 2.1}, {4.1, 7.2, 6.3}};
+
+int pick_bwd_split(const SplitCost& sc, double slices, int32_t nblk, const double (&walk)[3]) {
+  // the walks of the first, the middle and the last block
+  const double longest = std::fmax(walk[0], std::fmax(walk[1], walk[2])), mean = 0.25 * (walk[0] + 2.0 * walk[1] + walk[2]);
   int best = 0;
   double best_cost = 0.0;
-  for (int s = 0; s < kDkdvSplits; ++s) {
-    const DkdvSplit sp = kDkdvSplit[s];
-    const double unit = sp.kw / 4.0, n = (double)slices * nblk / unit;
-    const double alone = sp.kw * sp.qg == 8 ? 1.0 : 1.3;
+  for (int s = 0; s < kBwdSplits; ++s) {
+    const BwdSplit sp = kBwdSplit[s];
+    const double unit = sp.own / 4.0, n = slices * nblk / unit, fall = 2.0 * (longest - mean) * kCUs / n;
     double t = n * mean * unit / kCUs;
-    for (int k = 1; k <= 8 && (k - 1) * kCUs < n; ++k) {
-      const double len = longest - 2.0 * (longest - mean) * ((k - 1) * kCUs / n);
-      t = std::fmax(t, k * len * unit * (k == 1 ? alone : 1.0));
+    for (int k = 1; k <= 8 && (k == 1 || (k - 1) * kCUs < n); ++k) {
+      const double len = k * (longest - fall * (k - 1)) * unit * (k == 1 && sp.own * sp.groups == 4 ? sc.alone : 1.0);
+      t = t > len ? t : len;
     }
-    const double rounds = std::fmax(1.0, n / (sp.qg == 1 ? 2 * kCUs : kCUs));
-    const double cost = kPerStep[s] * t + (sp.qg == 1 ? 4.0 : 6.0) * rounds;
+    const double cost = sc.per_step[s] * t + sc.start[s] * std::fmax(1.0, n / (sp.groups == 1 ? 2 * kCUs : kCUs));
     if (s == 0 || cost < best_cost) {
       best = s;
       best_cost = cost;
     }
   }
   return best;
+}
+
+int pick_dkdv_split(const MaskSpec& m, int64_t slices, int64_t group, int32_t row_tile) {
+  const MaskGeom g = residue_geom(m, 0);
+  const int32_t nblk = (g.S + kBwdBlock - 1) / kBwdBlock;
+  auto walk = [&](int32_t blk) {
+    const RowSpan r = query_range(g, blk * kBwdBlock, imin32(blk * kBwdBlock + kBwdBlock - 1, g.S - 1));
+    return (double)group * (r.hi / row_tile - r.lo / row_tile + 1);
+  };
+  return pick_bwd_split(kDkdvCost, (double)slices, nblk, {walk(0), walk(nblk / 2), walk(nblk - 1)});
+}
+
+int pick_dq_split(const MaskSpec& m, int64_t slices, bool d64) {
+  const MaskGeom g = residue_geom(m, 0);
+  const int32_t nblk = (g.S + kBwdBlock - 1) / kBwdBlock;
+  auto walk = [&](int32_t blk) {
+    const TileRange t = tile_range(g, blk * kBwdBlock, imin32(blk * kBwdBlock + kBwdBlock - 1, g.S - 1), kBN);
+    return (double)(t.n_pre + t.n2);
+  };
+  return pick_bwd_split(d64 ? kDqCostD64 : kDqCostD128, (double)slices, nblk,
+                        {walk(0), walk(nblk / 2), walk(nblk - 1)});
 }
 
 hipError_t launch(BwdKernelFn fn, int64_t grid, int threads, const BwdParams& p, hipStream_t stream) {
@@ -631,8 +651,6 @@ int launch_bwd(const chia_attn_bwd_args* ba, void* stream, bool noalloc) {
   p.G = (int32_t)G;
   p.residues = num_residues(p.mask);
   p.SR = (int32_t)stats_rows(p.mask);
-  p.n_blk = (residue_geom(p.mask, 0).S + kBwdBlock - 1) / kBwdBlock;
-  p.div_blk = make_udiv(p.n_blk);
   p.div_res = make_udiv(p.residues);
   p.div_h = make_udiv(p.H);
   p.div_g = make_udiv(p.G);
@@ -643,8 +661,9 @@ int launch_bwd(const chia_attn_bwd_args* ba, void* stream, bool noalloc) {
   p.bias = a->bias;
   p.post_scale = a->post_scale;
 
-  const int64_t g_dq = a->batch * a->heads * p.residues * (int64_t)p.n_blk;
-  if (g_dq >= ((int64_t)1 << 31)) return CHIA_ATTN_ERR_SHAPE;
+  // (both kernels' grids: a split into 64-row blocks is chosen for small ones only)
+  const int64_t blocks = (residue_geom(p.mask, 0).S + kBwdBlock - 1) / kBwdBlock;
+  if (a->batch * a->heads * p.residues * blocks >= ((int64_t)1 << 31)) return CHIA_ATTN_ERR_SHAPE;
 
   const bool alibi = a->alibi_slopes != nullptr, softcap = a->softcap > 0.f;
   const BwdKernels ks = a->head_dim == 64 ? select_bwd_kernels_d64((int)a->norm, alibi, softcap)
@@ -657,17 +676,17 @@ int launch_bwd(const chia_attn_bwd_args* ba, void* stream, bool noalloc) {
   auto order_for = [&](int64_t heads) {
     return launch_order(zigzag_of(p.mask), a->batch * heads * p.residues, heads, p.residues, a->cu_seqlens != nullptr);
   };
-  p.order = order_for(a->heads);
-  err = launch(ks.dq, g_dq, 256, p, s);
-  p.order = order_for(hkv);
-  const int split = pick_dkdv_split(p.mask, a->batch * hkv * p.residues, G, a->head_dim == 64 ? 64 : 32);
-  const DkdvSplit sp = kDkdvSplit[split];
-  p.n_blk = (residue_geom(p.mask, 0).S + 32 * sp.kw - 1) / (32 * sp.kw);
-  p.div_blk = make_udiv(p.n_blk);
+  auto run = [&](BwdKernelFn fn, BwdSplit sp, int64_t heads) {
+    p.order = order_for(heads);
+    p.n_blk = (residue_geom(p.mask, 0).S + 32 * sp.own - 1) / (32 * sp.own);
+    p.div_blk = make_udiv(p.n_blk);
+    return launch(fn, a->batch * heads * p.residues * (int64_t)p.n_blk, 64 * sp.own * sp.groups, p, s);
+  };
+  const int dq = pick_dq_split(p.mask, a->batch * a->heads * p.residues, a->head_dim == 64);
+  err = run(ks.dq[dq], kBwdSplit[dq], a->heads);
+  const int dkdv = pick_dkdv_split(p.mask, a->batch * hkv * p.residues, G, a->head_dim == 64 ? 64 : 32);
   // a group whose query heads differ in scale takes c1 per score
-  const BwdKernelFn dkdv = ks.dkdv[split][G > 1 && a->head_scale ? 1 : 0];
-  if (err == hipSuccess)
-    err = launch(dkdv, a->batch * hkv * p.residues * (int64_t)p.n_blk, 64 * sp.kw * sp.qg, p, s);
+  if (err == hipSuccess) err = run(ks.dkdv[dkdv][G > 1 && a->head_scale ? 1 : 0], kBwdSplit[dkdv], hkv);
   return err == hipSuccess ? CHIA_ATTN_OK : (int)err;
 }
 }  // namespace

@@ -5,19 +5,19 @@
 namespace chia {
 
 template <int NORM, bool AL, bool SC, int SPLIT>
-static void set_dkdv(BwdKernels& k) {
-  constexpr int KW = kDkdvSplit[SPLIT].kw, QG = kDkdvSplit[SPLIT].qg;
-  k.dkdv[SPLIT][0] = attn_bwd_dkdv_kernel<128, NORM, AL, SC, false, KW, QG>;
-  k.dkdv[SPLIT][1] = attn_bwd_dkdv_kernel<128, NORM, AL, SC, true, KW, QG>;
+static void set_split(BwdKernels& k) {
+  constexpr int OWN = kBwdSplit[SPLIT].own, GROUPS = kBwdSplit[SPLIT].groups;
+  k.dq[SPLIT] = attn_bwd_dq_kernel<128, NORM, AL, SC, OWN, GROUPS>;
+  k.dkdv[SPLIT][0] = attn_bwd_dkdv_kernel<128, NORM, AL, SC, false, OWN, GROUPS>;
+  k.dkdv[SPLIT][1] = attn_bwd_dkdv_kernel<128, NORM, AL, SC, true, OWN, GROUPS>;
 }
 
 template <int NORM, bool AL, bool SC>
 static BwdKernels bwd_inst() {
   BwdKernels k;
-  k.dq = attn_bwd_dq_kernel<128, NORM, AL, SC>;
-  set_dkdv<NORM, AL, SC, 0>(k);
-  set_dkdv<NORM, AL, SC, 1>(k);
-  set_dkdv<NORM, AL, SC, 2>(k);
+  set_split<NORM, AL, SC, 0>(k);
+  set_split<NORM, AL, SC, 1>(k);
+  set_split<NORM, AL, SC, 2>(k);
   return k;
 }
 

@@ -216,8 +216,7 @@ __device__ __forceinline__ void dma_rows(const uint16_t* base, int64_t rs, int r
 // dma_rows with its per-lane offsets computed once for a fixed row stride: a
 // tile whose ROWS rows lie inside the sub-sequence adds only its uniform row
 // base, a 32 x 32 -> 64-bit product (rows are non-negative and a row step is
-// below 2^25 elements, so its byte count fits 32 bits); the last tile, whose
-// rows past the end are clamped, takes dma_rows.
+// below 2^25 elements, so its byte count fits 32 bits).
 template <int D, int NW, int ROWS = 64>
 struct RowDma {
   static constexpr int DQ = D / 8, NDMA = ROWS * DQ / (NW * 64);
@@ -236,15 +235,22 @@ struct RowDma {
       off[n] = (uint32_t)r * row_bytes + 16 * k_slot<D>(r, slot);
     }
   }
-  __device__ void operator()(const uint16_t* base, int64_t rs, int row, int S, char* dst, int wave, int lane) const {
+  __device__ void operator()(const uint16_t* base, int row, int S, char* dst, int wave, int lane) const {
+    const char* src = (const char*)base + (uint64_t)(uint32_t)row * row_bytes;
     if (row + ROWS <= S) {
-      const uint16_t* src = (const uint16_t*)((const char*)base + (uint64_t)(uint32_t)row * row_bytes);
 #pragma unroll
       for (int n = 0; n < NDMA; ++n)
-        dma16s((const char*)src + (uint64_t)(uint32_t)(n / ND * ND * RS) * row_bytes, off[n % ND],
+        dma16s(src + (uint64_t)(uint32_t)(n / ND * ND * RS) * row_bytes, off[n % ND],
                lds_addr(dst + (n * NW + wave) * 1024));
-    } else {
-      dma_rows<D, NW, ROWS>(base, rs, row, S, dst, wave, lane);
+    } else {  // the last tile: rows past the end clamped (its offsets from the row step alone,
+              // so that no 64-bit stride lives through the loop)
+#pragma unroll
+      for (int n = 0; n < NDMA; ++n) {
+        const int pos = (n * NW + wave) * 64 + lane;
+        const int r = pos / DQ, slot = pos % DQ;
+        const uint32_t rr = (uint32_t)imin32(r, S - 1 - row);
+        dma16s(src, rr * row_bytes + 16 * k_slot<D>(r, slot), lds_addr(dst + (n * NW + wave) * 1024));
+      }
     }
   }
 };
@@ -257,19 +263,19 @@ __device__ __forceinline__ uint32_t stage_behind(uint32_t cur) {
   return cur == 0 ? NS - 1 : cur - 1;
 }
 
-// Workgroup shapes of the dK/dV kernel: key wavefronts (32 keys each) times
-// query groups that split the walk over the query tiles.
-constexpr int kDkdvSplits = 3;
-struct DkdvSplit {
-  int kw, qg;
+// Workgroup shapes of both kernels: wavefronts that own 32 rows (dQ) or 32 keys
+// (dK/dV) each, times groups that split the walk over the key (query) tiles.
+constexpr int kBwdSplits = 3;
+struct BwdSplit {
+  int own, groups;
 };
-constexpr DkdvSplit kDkdvSplit[kDkdvSplits] = {{4, 1}, {4, 2}, {2, 4}};
+constexpr BwdSplit kBwdSplit[kBwdSplits] = {{4, 1}, {4, 2}, {2, 4}};
 
 // Kernel set of one (head_dim, normaliser, ALiBi, softcap) instantiation.
 using BwdKernelFn = void (*)(BwdParams);
 struct BwdKernels {
-  BwdKernelFn dq;
-  BwdKernelFn dkdv[kDkdvSplits][2];  // [split][1: a K/V group's heads differ in scale]
+  BwdKernelFn dq[kBwdSplits];
+  BwdKernelFn dkdv[kBwdSplits][2];  // [split][1: a K/V group's heads differ in scale]
 };
 
 // do . o over the 8 DK bf16 values of one lane's half row (chunks 16 kk + 8 lh
@@ -289,24 +295,57 @@ __device__ __forceinline__ float half_row_dot(const bf16x8_t* x, const bf16x8_t*
   return acc;
 }
 
+// The sums of NG groups of NW wavefronts meet in LDS: groups 1 .. NG - 1 write
+// theirs lane-major over the stages, group 0 adds them in group order.
+template <int DB, int NG, int NW, int LDS_BYTES>
+__device__ __forceinline__ void add_groups(f32x16_t* acc, float* mb, int grp, int wave, int lane) {
+  constexpr int FL = 16 * DB * 64;  // floats of one wavefront
+  static_assert((NG - 1) * NW * FL * 4 <= LDS_BYTES, "the sums fit the stages");
+  __syncthreads();  // every wavefront is past its last read of the stages
+  if (grp > 0) {
+    float* dst = mb + ((grp - 1) * NW + wave) * FL + lane;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) dst[(16 * db + e) * 64] = acc[db][e];
+  }
+  __syncthreads();
+  if (grp == 0) {
+#pragma unroll
+    for (int q = 0; q < NG - 1; ++q) {
+      const float* src = mb + (q * NW + wave) * FL + lane;
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[db][e] += src[(16 * db + e) * 64];
+    }
+  }
+}
 
 // ---- dQ ------------------------------------------------------------------------
-template <int D, int NORM, bool ALIBI, bool SOFTCAP>
-__global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(const BwdParams p) {
-  constexpr int NW = 4, BN = 64, KB = BN / 32, DK = D / 16, DB = D / 32;
+// RW: row wavefronts, 32 query rows each.  KG: key groups of RW wavefronts that
+// split the walk over the key tiles (as dK/dV's query groups; four groups take
+// 32-key tiles, so that their stages fit).
+template <int D, int NORM, bool ALIBI, bool SOFTCAP, int RW, int KG>
+__global__ __launch_bounds__(64 * RW * KG, 2) void attn_bwd_dq_kernel(const BwdParams p) {
+  constexpr int NW = RW, BN = KG == 4 ? 32 : 64, KB = BN / 32, DK = D / 16, DB = D / 32;
+  constexpr int BR = 32 * RW;  // rows per workgroup
   constexpr int RP = 2 * D, T_BYTES = BN * RP, STAGE_BYTES = 2 * T_BYTES;
-  constexpr int NS = D == 64 ? 3 : 2;
-  __shared__ __attribute__((aligned(1024))) char lds[NS * STAGE_BYTES];
+  constexpr int NS = D == 64 && KG == 1 ? 3 : 2;
+  __shared__ __attribute__((aligned(1024))) char lds_all[KG * NS * STAGE_BYTES];
 
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave_wg = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = KG > 1 ? wave_wg / RW : 0;         // this wavefront's key group
+  const int wave = KG > 1 ? wave_wg % RW : wave_wg;  // and its index in the group
+  char* const lds = lds_all + grp * (NS * STAGE_BYTES);  // the group's stages
   const int lq = lane & 31, lh = lane >> 5;
 
   // workgroup -> (b, h, residue, 128-row block), heaviest blocks first
   // (packed sequences of unequal length: round-robin over the XCDs, no remap)
   // the query blocks with the most keys first
   int bhr, blk;
-  if (p.order.slices > 0) {
+  if (p.order.hx > 0) {
     const SliceUnit su = rank_order((int)blockIdx.x, p.order, p.n_blk);
     bhr = su.slice;
     blk = su.unit;
@@ -322,7 +361,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(const BwdParams p) 
   MaskSpec ms = p.mask;
   ms.S = seq.len;
   const MaskGeom g = residue_geom(ms, r);
-  const int nblk_r = (g.S + 127) / 128;
+  const int nblk_r = (g.S + BR - 1) / BR;
   if (blk >= nblk_r) return;  // whole workgroup, before any barrier
   const int hkv = udiv(h, p.div_g);
   const int dil = p.mask.dil;
@@ -338,11 +377,13 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(const BwdParams p) 
   // scores it with the plain (unbiased) formulas.
   constexpr bool kSeed = ALIBI && !SOFTCAP;
   ScoreGrad<NORM, ALIBI && !kSeed, SOFTCAP> sg = score_consts<NORM, ALIBI && !kSeed, SOFTCAP>(p);
-  sg.set_head(p.scale * (p.head_scale ? p.head_scale[h] : 1.0f),
-              (ALIBI && p.alibi_slopes) ? p.alibi_slopes[h] * (float)dil : 0.0f);
+  const float hc1 = p.scale * (p.head_scale ? p.head_scale[h] : 1.0f);
+  const float hsl = (ALIBI && p.alibi_slopes) ? p.alibi_slopes[h] * (float)dil : 0.0f;
+  if constexpr (D == 64) sg.set_head(hc1, hsl);
+  else sg.set_head(uniform_f(hc1), uniform_f(hsl));  // (no vector register to spare)
 
   // this wavefront's 32 rows: Q and dO as MFMA B operands (lane = row)
-  const int row0 = blk * 128 + 32 * wave;
+  const int row0 = blk * BR + 32 * wave;
   const int i = row0 + lq;
   const bool ok = i < g.S;
   bf16x8_t qf[DK], df[DK];
@@ -366,9 +407,13 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(const BwdParams p) 
   }
 
   // key tiles of the workgroup's rows; per-wavefront classification bounds
-  const int wg_hi = imin32(blk * 128 + 127, g.S - 1);
-  const TileRange tr = tile_range(g, blk * 128, wg_hi, BN);
-  const int ntiles = tr.n_pre + tr.n2;
+  const int wg_hi = imin32(blk * BR + BR - 1, g.S - 1);
+  const TileRange tr = tile_range(g, blk * BR, wg_hi, BN);
+  // this group's tiles (tile t belongs to group t % KG), and the steps of the
+  // group with the most
+  const int n_all = tr.n_pre + tr.n2;
+  const int ntiles = KG == 1 ? n_all : (n_all - grp + KG - 1) / KG;
+  const int nsteps = KG == 1 ? n_all : (n_all + KG - 1) / KG;
   const bool wvalid = row0 < g.S;
   const int ra = row0, rb = imin32(row0 + 31, g.S - 1);
 
@@ -391,16 +436,17 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(const BwdParams p) 
   // stage is a wrapping counter; the class comes from per-wavefront bounds
   // (mask.h); the DMA's per-lane offsets are fixed once.
   const int seam = tr.n_pre;
-  const RowDma<D, NW> kdma(krs, wave, lane), vdma(vrs, wave, lane);
+  const RowDma<D, NW, BN> kdma(krs, wave, lane), vdma(vrs, wave, lane);
+  auto first_key = [&](int it) { return tile_at(tr, KG == 1 ? it : grp + it * KG) * BN; };
   auto issue = [&](int jt0, uint32_t stage) {
     char* st = lds + stage * STAGE_BYTES;
-    kdma(kh, krs, jt0, g.S, st, wave, lane);
-    vdma(vh, vrs, jt0, g.S, st + T_BYTES, wave, lane);
+    kdma(kh, jt0, g.S, st, wave, lane);
+    vdma(vh, jt0, g.S, st + T_BYTES, wave, lane);
   };
-  constexpr int NDMA2 = 2 * (64 * (D / 8) / (NW * 64));  // loads per tile per wavefront
+  constexpr int NDMA2 = 2 * (BN * (D / 8) / (NW * 64));  // loads per tile per wavefront
   int dma_next = 0, jt_dma = 0;
   for (; dma_next < NS - 1 && dma_next < ntiles; ++dma_next) {
-    jt_dma = (dma_next == 0 || dma_next == seam) ? tile_at(tr, dma_next) * BN : jt_dma + BN;
+    jt_dma = (KG > 1 || dma_next == 0 || dma_next == seam) ? first_key(dma_next) : jt_dma + BN;
     issue(jt_dma, (uint32_t)dma_next);
   }
   const KeyRanges<BN> kr(g, wvalid, ra, rb);
@@ -417,7 +463,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(const BwdParams p) 
     lse2 = p.lse[b * p.lse_sb + h * p.lse_sh + (t0 + (int64_t)(ok ? i : 0) * dil) * p.lse_ss] * kLog2e;
     const float part = half_row_dot<DK>(df, of);
     ndelta = -(part + __shfl_xor(part, 32));
-    if (ok && lh == 0) {
+    if (ok && lh == 0 && grp == 0) {
       const int64_t o2 = ((int64_t)(b * p.H + h) * p.residues + r) * p.SR + i;  // b: the sequence
       p.stats[o2] = lse2;
       p.stats[(int64_t)p.B * p.H * p.residues * p.SR + o2] = ndelta;
@@ -426,7 +472,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(const BwdParams p) 
   }
 
   typedef short i16x8_t __attribute__((ext_vector_type(8)));
-  for (int it = 0; it < ntiles; ++it) {
+  for (int it = 0; it < nsteps; ++it) {
     if (dma_next - (it + 1) >= 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA2) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -434,12 +480,13 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(const BwdParams p) 
     const uint32_t st_it = st_cur;  // it mod NS
     st_cur = st_it + 1 == NS ? 0 : st_it + 1;
     if (dma_next < ntiles) {
-      jt_dma = dma_next == seam ? tile_at(tr, dma_next) * BN : jt_dma + BN;
+      jt_dma = (KG > 1 || dma_next == seam) ? first_key(dma_next) : jt_dma + BN;
       issue(jt_dma, stage_behind<NS>(st_it));
       ++dma_next;
     }
+    if (KG > 1 && it >= ntiles) break;  // (the last step, in a group with one tile fewer)
     const char* St = lds + st_it * STAGE_BYTES;
-    jt0 = (it == 0 || it == seam) ? tile_at(tr, it) * BN : jt0 + BN;
+    jt0 = (KG > 1 || it == 0 || it == seam) ? first_key(it) : jt0 + BN;
     const int cls = key_class(kr, jt0);
     if (cls == TILE_EMPTY) continue;
 
@@ -489,6 +536,11 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(const BwdParams p) 
         dq[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, __builtin_bit_cast(bf16x8_t, wv), dq[db], 0, 0, 0);
       }
     }
+  }
+
+  if constexpr (KG > 1) {
+    add_groups<DB, KG, RW, sizeof(lds_all)>(dq, reinterpret_cast<float*>(lds_all), grp, wave, lane);
+    if (grp > 0) return;
   }
 
   if (ok) {
@@ -544,7 +596,7 @@ __global__ __launch_bounds__(64 * KW * QG, 2) void attn_bwd_dkdv_kernel(const Bw
   // the key blocks with the most queries (the first ones) first
   int bhr, blk = 0;
   int unit = -1;  // longest-first: blocks counted from the sequence's last one
-  if (p.order.slices > 0) {
+  if (p.order.hx > 0) {
     const SliceUnit su = rank_order((int)blockIdx.x, p.order, p.n_blk);
     bhr = su.slice;
     unit = su.unit;
@@ -672,8 +724,8 @@ __global__ __launch_bounds__(64 * KW * QG, 2) void attn_bwd_dkdv_kernel(const Bw
   auto issue = [&](uint32_t stage) {
     const int i0 = dc.qt * BM;
     char* st = lds + stage * STAGE_BYTES;
-    qdma(dc.qb, qrs, i0, g.S, st, wave, lane);
-    dodma(dc.dob, dors, i0, g.S, st + T_BYTES, wave, lane);
+    qdma(dc.qb, i0, g.S, st, wave, lane);
+    dodma(dc.dob, i0, g.S, st + T_BYTES, wave, lane);
     if constexpr (kStats) {
       // the group's first KW / 2 wavefronts move lse log2 e, the others -delta,
       // SN rows each; the stats rows are padded to 64
@@ -810,34 +862,8 @@ __global__ __launch_bounds__(64 * KW * QG, 2) void attn_bwd_dkdv_kernel(const Bw
   }
 
   if constexpr (QG > 1) {
-    // the groups' sums meet in LDS, dK and then dV: groups 1 .. QG - 1 write
-    // theirs lane-major over the stages, group 0 adds them in group order
-    constexpr int FL = 16 * DB * 64;  // floats of one wavefront's dK or dV
-    static_assert((QG - 1) * KW * FL * 4 <= (int)sizeof(lds_all), "the sums fit the stages");
-    float* const mb = reinterpret_cast<float*>(lds_all);
-    auto merge = [&](f32x16_t* acc) __attribute__((always_inline)) {
-      __syncthreads();  // every wavefront is past its last read of the stages
-      if (grp > 0) {
-        float* dst = mb + ((grp - 1) * KW + wave) * FL + lane;
-#pragma unroll
-        for (int db = 0; db < DB; ++db)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) dst[(16 * db + e) * 64] = acc[db][e];
-      }
-      __syncthreads();
-      if (grp == 0) {
-#pragma unroll
-        for (int q = 0; q < QG - 1; ++q) {
-          const float* src = mb + (q * KW + wave) * FL + lane;
-#pragma unroll
-          for (int db = 0; db < DB; ++db)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[db][e] += src[(16 * db + e) * 64];
-        }
-      }
-    };
-    merge(dk);
-    merge(dv);
+    add_groups<DB, QG, KW, sizeof(lds_all)>(dk, reinterpret_cast<float*>(lds_all), grp, wave, lane);
+    add_groups<DB, QG, KW, sizeof(lds_all)>(dv, reinterpret_cast<float*>(lds_all), grp, wave, lane);
     if (grp > 0) return;
   }
 

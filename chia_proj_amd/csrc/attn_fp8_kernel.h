@@ -125,7 +125,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_fp8_kernel(const Fp8Params p)
   // to last, ... (LaunchOrder).  Otherwise each XCD gets a contiguous range of slices, longest block first
   // per slice; packed sequences go round-robin to the XCDs.
   int bhr, blk;
-  if (p.order.slices > 0) {
+  if (p.order.hx > 0) {
     const SliceUnit su = rank_order((int)blockIdx.x, p.order, p.n_blk);
     bhr = su.slice;
     blk = su.unit;

@@ -108,7 +108,7 @@ __global__ __launch_bounds__(64 * RW * NG * KG, Q1Config<D>::occupancy) void att
 
   // ---- workgroup -> (batch, head, residue, unit) ----------------------------
   int bhr, pr;
-  if (p.order.slices > 0) {
+  if (p.order.hx > 0) {
     const SliceUnit su = rank_order((int)blockIdx.x, p.order, p.n_pairs);
     bhr = su.slice;
     pr = su.unit;

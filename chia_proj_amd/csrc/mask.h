@@ -369,45 +369,39 @@ CHIA_HD MaskGeom residue_geom(const MaskSpec& m, int32_t r) {
 // across sequences of unequal length (the units a sequence does not have exit
 // at once).
 //
-// hx > 0: XCD x (workgroups x, x + 8, ...) serves hx slices, so that a slice's
-// K and V stay in one L2: heads [x hh, (x + 1) hh) of every hs consecutive
-// slices.  A fixed-length launch takes one run of all its slices (hh = hx);
-// packed sequences a run per sequence, as unequal sequences would otherwise
-// leave the XCDs unequal work.  hx = 0 (counts that do not divide by 8): the
-// slices of a rank go round the XCDs.  slices = 0: the order is off.
+// shift = 3: XCD x (workgroups x, x + 8, ...) serves hx slices, so that a
+// slice's K and V stay in one L2: heads [x hh, (x + 1) hh) of every hs
+// consecutive slices.  A fixed-length launch takes one run of all its slices
+// (hh = hx); packed sequences a run per sequence, as unequal sequences would
+// otherwise leave the XCDs unequal work.  shift = 0 (counts that do not divide
+// by 8): the slices of a rank go round the XCDs (one run, hh = hx = all
+// slices).  hx = 0: the order is off.
 struct LaunchOrder {
-  int32_t slices, hx, hh, hs;
-  UDiv div_slices, div_hx, div_hh;
+  int32_t shift, hx, hh, hs;
+  UDiv div_hx, div_hh;
 };
 struct SliceUnit {
   int slice, unit;
 };
 // Bijective between the slices * n_units workgroups and (slice, unit).
 CHIA_HD SliceUnit rank_order(int x, const LaunchOrder& o, int n_units) {
-  if (o.hx > 0) {
-    const int xcd = x & 7, local = x >> 3;
-    const int rank = udiv(local, o.div_hx), s = local - rank * o.hx, run = udiv(s, o.div_hh);
-    return SliceUnit{run * o.hs + xcd * o.hh + (s - run * o.hh), n_units - 1 - rank};
-  }
-  const int rank = udiv(x, o.div_slices);
-  return SliceUnit{x - rank * o.slices, n_units - 1 - rank};
+  const int xcd = x & ((1 << o.shift) - 1), local = x >> o.shift;
+  const int rank = udiv(local, o.div_hx), s = local - rank * o.hx, run = udiv(s, o.div_hh);
+  return SliceUnit{run * o.hs + xcd * o.hh + (s - run * o.hh), n_units - 1 - rank};
 }
 
 // The longest-first order over `slices` (batch, head, residue) slices
 // of `heads` heads, or the natural one when `on` is false.
 inline LaunchOrder launch_order(bool on, int64_t slices, int64_t heads, int64_t residues, bool packed) {
-  LaunchOrder o{0, 0, 1, 0, make_udiv(1), make_udiv(1), make_udiv(1)};
+  LaunchOrder o{0, 0, 1, 0, make_udiv(1), make_udiv(1)};
   if (!on) return o;
-  o.slices = (int32_t)slices;
-  o.div_slices = make_udiv(o.slices);
   const bool per_seq = packed && residues == 1 && heads % 8 == 0;
-  if (per_seq || (!packed && slices % 8 == 0)) {
-    o.hx = (int32_t)(slices / 8);
-    o.hh = per_seq ? (int32_t)(heads / 8) : o.hx;
-    o.hs = per_seq ? (int32_t)heads : 0;
-    o.div_hx = make_udiv(o.hx);
-    o.div_hh = make_udiv(o.hh);
-  }
+  o.shift = per_seq || (!packed && slices % 8 == 0) ? 3 : 0;
+  o.hx = (int32_t)(slices >> o.shift);
+  o.hh = per_seq ? (int32_t)(heads / 8) : o.hx;
+  o.hs = per_seq ? (int32_t)heads : 0;
+  o.div_hx = make_udiv(o.hx);
+  o.div_hh = make_udiv(o.hh);
   return o;
 }
 

@@ -23,7 +23,7 @@ int main(int argc, char** argv) {
           for (bool packed : {false, true}) {
             const int slices = batch * heads * res;
             LaunchOrder o = launch_order(true, slices, heads, res, packed);
-            if (planted && o.hx > 0 && packed) o.hs -= 1;  // neighbouring runs overlap
+            if (planted && o.shift == 3 && packed) o.hs -= 1;  // neighbouring runs overlap
             std::vector<char> seen((size_t)slices * units, 0);
             std::map<int, int> xcd_of;
             std::map<std::pair<int, int>, int> per_xcd;  // (XCD, sequence) -> slices
@@ -36,13 +36,13 @@ int main(int argc, char** argv) {
               if (s++) ++bad;
               if (x % 8 == 0 && su.unit > last) ++bad;
               if (x % 8 == 0) last = su.unit;
-              if (o.hx > 0) {
+              if (o.shift == 3) {
                 if (xcd_of.count(su.slice) && xcd_of[su.slice] != x % 8) ++bad;
                 if (!xcd_of.count(su.slice)) ++per_xcd[{x % 8, packed ? su.slice / heads : 0}];
                 xcd_of[su.slice] = x % 8;
               }
             }
-            if (o.hx > 0) {
+            if (o.shift == 3) {
               const int each = packed ? heads / 8 : slices / 8;
               for (auto& kv : per_xcd)
                 if (kv.second != each) ++bad;

@@ -152,6 +152,31 @@ def test_backward_query_groups(name, B, H, Hkv, S, D, kw):
         _check(f"{name} b={b} hk={hk}", [grads[0][b:b + 1, hq]] + [g[b:b + 1, hk:hk + 1] for g in grads[1:]], refs)
 
 
+# dQ's key groups: four groups of 32-key tiles on two heads (from one tile to ragged counts), and
+# two groups where 64 to 128 blocks of equal, long walks leave CUs idle.
+DQ_SPLIT = [
+    *[(f"four_groups_{n}_S{S}_d{D}", 1, 2, S, D, kw) for D in (64, 128) for S in (40, 95, 129, 700)
+      for n, kw in (("causal", dict(causal=True)), ("prefix", dict(causal=True, prefix=50)),
+                    ("alibi_softcap", dict(causal=True, softcap=20.0, alibi_slopes=[0.1, 0.01])))],
+    *[(f"two_groups_{n}_d{D}", 1, 16, 1000, D, kw) for D in (64, 128) for n, kw in (
+        ("full", dict(causal=False)), ("relu", dict(causal=False, norm="relu", post_scale=0.01)))],
+]
+
+
+@pytest.mark.parametrize("name,B,H,S,D,kw", DQ_SPLIT, ids=[e[0] for e in DQ_SPLIT])
+def test_backward_key_groups(name, B, H, S, D, kw):
+    _say(f"[bwd] dq split {name}")
+    q, k, v, do = _draw(B, H, H, S, D, 7000 + S + D)
+    _, grads = _run(q, k, v, do, lambda a, b, c: attention(a, b, c, **kw))
+    for h in {0, H - 1}:
+        part = dict(kw)
+        if "alibi_slopes" in kw:
+            part["alibi_slopes"] = kw["alibi_slopes"][h:h + 1]
+        hs = slice(h, h + 1)
+        refs = attention_grad_ref(q[:, hs], k[:, hs], v[:, hs], do[:, hs], **part)
+        _check(f"{name} h={h}", [g[:, hs] for g in grads], refs)
+
+
 def test_backward_causal_s2048_sampled_heads():
     """B2 H4 S2048 D64 causal softmax: the full kernel grid, two heads checked."""
     _say("[bwd] causal S2048")

@@ -594,7 +594,7 @@ def attention_fp8_varlen(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_s
     if T == 0:
         check_cu_seqlens(cu_seqlens, 0, max_seqlen)
         return torch.empty(q.shape, dtype=torch.bfloat16, device=q.device) if out is None else out
-    B, S, cu, order = _cu_plan(cu_seqlens, T, max_seqlen, q.device)
+    B, S, cu, order, _ = _cu_plan(cu_seqlens, T, max_seqlen, q.device)
     sc = _check_params(D, norm, window, dilation, block, prefix, scale, softcap)
 
     def layout_ok(t):
@@ -673,11 +673,13 @@ _cu_cache: "OrderedDict[tuple, tuple]" = OrderedDict()
 
 
 def _cu_plan(cu_seqlens, total: int, max_seqlen: Optional[int], device):
-    """(B, max length, int32 device offsets, device dispatch order) for a checked
-    cu_seqlens.  The check reads the offsets on the host (a device tensor: one
+    """(B, max length, int32 device offsets, device dispatch order, work) for a
+    checked cu_seqlens.  The check reads the offsets on the host (a device tensor: one
     synchronisation); the result is cached per tensor storage and version, so a
     cu_seqlens reused unchanged (every layer of a model) is checked once.  The
-    order puts the longest sequences first (a shorter tail of the launch)."""
+    order puts the longest sequences first (a shorter tail of the launch); work
+    is the sum of the squared lengths / max length, a multiple of 8 (what the
+    argument struct's q batch stride says of a packed batch)."""
     key = None
     if isinstance(cu_seqlens, torch.Tensor) and not torch.compiler.is_compiling():
         # the same live tensor object (a weak reference guards against a new
@@ -691,7 +693,8 @@ def _cu_plan(cu_seqlens, total: int, max_seqlen: Optional[int], device):
     host, lens, longest = _host_cu_seqlens(cu_seqlens, total, max_seqlen)
     order = np.argsort(-lens, kind="stable")
     both = torch.from_numpy(np.concatenate((host, order)).astype(np.int32)).to(device)  # one copy
-    out = (len(lens), longest, both[:len(host)], both[len(host):])
+    work = -(-int((lens * lens).sum()) // (8 * max(longest, 1))) * 8
+    out = (len(lens), longest, both[:len(host)], both[len(host):], work)
     if key is not None:
         _cu_cache[key] = (weakref.ref(cu_seqlens), out)
         if len(_cu_cache) > _CU_CACHE_MAX:
@@ -714,7 +717,7 @@ def _prepare_varlen(q, k, v, cu_seqlens, max_seqlen, out, *, norm, causal, windo
         raise TypeError(f"q, k, v must be bfloat16, got {q.dtype}, {k.dtype}, {v.dtype}")
     if q.device.type != "cuda" or k.device != q.device or v.device != q.device:
         raise ValueError(f"q, k, v must be on the same GPU device, got {q.device}, {k.device}, {v.device}")
-    B, S, cu, order = _cu_plan(cu_seqlens, T, max_seqlen, q.device)
+    B, S, cu, order, work = _cu_plan(cu_seqlens, T, max_seqlen, q.device)
     sc = _check_params(D, norm, window, dilation, block, prefix, scale, softcap)
     q_, k_, v_ = (t if _layout_ok_packed(t) else t.contiguous() for t in (q, k, v))
     if out is None:
@@ -733,6 +736,7 @@ def _prepare_varlen(q, k, v, cu_seqlens, max_seqlen, out, *, norm, causal, windo
     for name, t in (("q_stride", q_), ("k_stride", k_), ("v_stride", v_), ("o_stride", o)):
         st = getattr(a, name)
         st[0], st[1], st[2] = 0, t.stride(1), t.stride(0)
+    a.q_stride[0] = work
     a.head_scale = hs.data_ptr() if hs is not None else None
     a.alibi_slopes = sl.data_ptr() if sl is not None else None
     a.cu_seqlens = cu.data_ptr()

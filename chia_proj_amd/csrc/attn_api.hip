@@ -73,6 +73,15 @@ int validate(const chia_attn_args* a, bool need_tensors) {
 // first token; the batch stride is not used.
 int64_t batch_stride(const chia_attn_args* a, const int64_t* st) { return a->cu_seqlens ? 0 : st[0]; }
 
+// The work of packed sequences as a share of `batch` sequences of seqlen
+// tokens, from the hint in q_stride[0] (header), or `unknown` without one.  It
+// chooses between launch shapes only.
+double packed_share(const chia_attn_args* a, double unknown) {
+  if (!a->cu_seqlens) return 1.0;
+  const double most = (double)a->batch * (double)a->seqlen, hint = (double)a->q_stride[0];
+  return hint > 0.0 && hint < most + 8.0 ? std::fmin(hint / most, 1.0) : unknown;
+}
+
 MaskSpec spec_of(const chia_attn_args* a) {
   return make_mask_spec((int32_t)a->seqlen, a->causal ? 1 : 0, a->window, a->dilation, a->block, a->prefix);
 }
@@ -257,11 +266,12 @@ Geometry launch_geometry(const chia_attn_args* a, const MaskSpec& m, const Score
   const bool banded = m.hi < kInf || m.blk > 0, causal = zigzag_of(m), softmax = a->norm == CHIA_ATTN_NORM_SOFTMAX;
   const MaskGeom g = residue_geom(m, 0);
   const int32_t nblk = (g.S + 127) / 128;
-  // Packed sequences: the launch is sized for the longest one and their lengths
-  // are not known here; the others are taken to add up to what makes 0.4 (0.5)
-  // of the grid real, and banded masks keep one block per workgroup.
+  // Packed sequences: the launch is sized for the longest one; the share of it
+  // that is real is the caller's hint, or taken to be 0.4 (0.5) (16 heads D64,
+  // ALiBi, 2025 + 126 + 573 + 64 + 133 + 3259 + 424 + 1854 tokens: 103 us with
+  // 0.4, 83 with the true 0.22, which takes more key groups).  Banded masks keep one block per workgroup.
   const bool packed = a->cu_seqlens != nullptr;
-  const double slices = (double)(a->batch * a->heads * geo.residues) * (!packed ? 1.0 : d64 ? 0.4 : 0.5);
+  const double slices = (double)(a->batch * a->heads * geo.residues) * packed_share(a, d64 ? 0.4 : 0.5);
   // Causal softmax at head_dim 64 whose pairs are exactly one round of two
   // workgroups per CU, of whole tiles: every CU ends at the same time and the
   // pairs stay (B1 H16 S8192: 154.7 against 163.3 us, ALiBi 154 against 163;
@@ -498,24 +508,24 @@ int pick_bwd_split(const SplitCost& sc, double slices, int32_t nblk, const doubl
   return best;
 }
 
-int pick_dkdv_split(const MaskSpec& m, int64_t slices, int64_t group, int32_t row_tile) {
+int pick_dkdv_split(const MaskSpec& m, double slices, int64_t group, int32_t row_tile) {
   const MaskGeom g = residue_geom(m, 0);
   const int32_t nblk = (g.S + kBwdBlock - 1) / kBwdBlock;
   auto walk = [&](int32_t blk) {
     const RowSpan r = query_range(g, blk * kBwdBlock, imin32(blk * kBwdBlock + kBwdBlock - 1, g.S - 1));
     return (double)group * (r.hi / row_tile - r.lo / row_tile + 1);
   };
-  return pick_bwd_split(kDkdvCost, (double)slices, nblk, {walk(0), walk(nblk / 2), walk(nblk - 1)});
+  return pick_bwd_split(kDkdvCost, slices, nblk, {walk(0), walk(nblk / 2), walk(nblk - 1)});
 }
 
-int pick_dq_split(const MaskSpec& m, int64_t slices, bool d64) {
+int pick_dq_split(const MaskSpec& m, double slices, bool d64) {
   const MaskGeom g = residue_geom(m, 0);
   const int32_t nblk = (g.S + kBwdBlock - 1) / kBwdBlock;
   auto walk = [&](int32_t blk) {
     const TileRange t = tile_range(g, blk * kBwdBlock, imin32(blk * kBwdBlock + kBwdBlock - 1, g.S - 1), kBN);
     return (double)(t.n_pre + t.n2);
   };
-  return pick_bwd_split(d64 ? kDqCostD64 : kDqCostD128, (double)slices, nblk,
+  return pick_bwd_split(d64 ? kDqCostD64 : kDqCostD128, slices, nblk,
                         {walk(0), walk(nblk / 2), walk(nblk - 1)});
 }
 
@@ -682,9 +692,10 @@ int launch_bwd(const chia_attn_bwd_args* ba, void* stream, bool noalloc) {
     p.div_blk = make_udiv(p.n_blk);
     return launch(fn, a->batch * heads * p.residues * (int64_t)p.n_blk, 64 * sp.own * sp.groups, p, s);
   };
-  const int dq = pick_dq_split(p.mask, a->batch * a->heads * p.residues, a->head_dim == 64);
+  const double slices = (double)(a->batch * p.residues) * packed_share(a, 1.0);
+  const int dq = pick_dq_split(p.mask, slices * (double)a->heads, a->head_dim == 64);
   err = run(ks.dq[dq], kBwdSplit[dq], a->heads);
-  const int dkdv = pick_dkdv_split(p.mask, a->batch * hkv * p.residues, G, a->head_dim == 64 ? 64 : 32);
+  const int dkdv = pick_dkdv_split(p.mask, slices * (double)hkv, G, a->head_dim == 64 ? 64 : 32);
   // a group whose query heads differ in scale takes c1 per score
   if (err == hipSuccess) err = run(ks.dkdv[dkdv][G > 1 && a->head_scale ? 1 : 0], kBwdSplit[dkdv], hkv);
   return err == hipSuccess ? CHIA_ATTN_OK : (int)err;

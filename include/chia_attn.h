@@ -114,8 +114,12 @@ typedef struct chia_attn_args {
    * seqlen tokens and the tensors are [B, H, S, D] as above.  Otherwise a
    * device int32[batch + 1] with cu_seqlens[0] = 0, non-decreasing: sequence b
    * is tokens [cu_seqlens[b], cu_seqlens[b + 1]) of packed tensors q, o
-   * [T, H, D] and k, v [T, H_kv, D]; the batch strides (stride[0]) are ignored
-   * and stride[2] steps one token.  seqlen must be >= every sequence's length
+   * [T, H, D] and k, v [T, H_kv, D]; the batch strides (stride[0]) address
+   * nothing and stride[2] steps one token.  q_stride[0] may say how much of the
+   * work is there: the sum of the squared lengths / seqlen, rounded up to a
+   * multiple of 8 (equal lengths: the total of tokens).  It only helps to choose
+   * the launch shape; a value outside (0, batch * seqlen + 8) is
+   * ignored.  seqlen must be >= every sequence's length
    * (rows beyond seqlen are not computed).  Masks and ALiBi positions count
    * from each sequence's first token.  The values are read by the GPU and not
    * checked: the caller guarantees them (the Python layer checks a host copy).

@@ -231,7 +231,9 @@ def _backward_varlen(ctx, do, _dlse):
     q, k, v, o, lse, cu_seqlens = ctx.saved_tensors
     if do is None:
         return (None,) * (4 + len(ctx.rest))
-    if _traced(do):
+    # grad mode is on here only under create_graph=True: the operator, which has no
+    # second derivative, then refuses one instead of leaving it out of a sum
+    if _traced(do) or torch.is_grad_enabled():
         dq, dk, dv = torch.ops.chia_attn.bwd_varlen(do, q, k, v, o, lse, cu_seqlens, *ctx.rest)
     else:
         from .attention import run_backward_varlen

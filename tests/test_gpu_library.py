@@ -282,3 +282,21 @@ def test_eager_training_leaves_transforms_to_the_operator():
     assert any("chia_attn.fwd" in n for n in mode.names)
     with pytest.raises(RuntimeError):  # torch.func.grad through a custom operator: refused by torch
         torch.func.grad(lambda a: attention(a, k.detach(), v.detach()).float().sum())(q.detach())
+
+
+def test_packed_second_derivative_is_refused():
+    """create_graph=True gives the same gradients, and a loss with a term through them is
+    refused (the packed backward has no derivative of its own), not silently cut short."""
+    from chia_proj_amd import attention_varlen
+
+    _say("[lib] packed create_graph")
+    cu = torch.tensor([0, 50, 96], dtype=torch.int32, device=DEV)
+    ts = [t[0].transpose(0, 1).contiguous().requires_grad_(True) for t in _qkv(1, 2, 2, 96, 64, seed=4)]
+    o = attention_varlen(*ts, cu, 50, causal=True)
+    do = torch.ones_like(o)
+    want = torch.autograd.grad(o, ts, do, retain_graph=True)
+    got = torch.autograd.grad(o, ts, do, create_graph=True)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    with pytest.raises(RuntimeError):
+        (got[0].float().sum() + ts[0].float().sum()).backward()

@@ -119,6 +119,7 @@ struct Geometry {
   int shape;       // one-block core: the workgroup's shape (Q1Shape)
   int groups;      // and its groups of `waves` wavefronts
   bool rank;       // launch the units with the most keys first (rank_order)
+  bool fixed_ref;  // softcap softmax may take its weights against the fixed reference (cap_fixed)
   int64_t workgroups;
 };
 
@@ -130,7 +131,7 @@ Geometry paired_geometry(const MaskSpec& m, int64_t batch, int64_t heads) {
   geo.q1 = false;
   geo.shape = Q1_ONE;
   geo.groups = 1;
-  geo.rank = false;
+  geo.rank = geo.fixed_ref = false;
   const int32_t s0 = residue_geom(m, 0).S;  // longest residue class
   // 4 wavefronts share each K/V tile among more rows; fall back to 2 when
   // that leaves fewer than two workgroups per CU.  Windowed or block masks
@@ -203,7 +204,7 @@ Geometry plan_geometry(const chia_attn_args* a, const MaskSpec& m, const ScorePa
   if (a->head_dim == 128 && a->norm != CHIA_ATTN_NORM_SOFTMAX && !geo.zigzag && !banded && s0 >= 2048 && !sp.alibi &&
       !sp.softcap && geo.waves == 4)
     return geo;
-  geo.q1 = true;
+  geo.q1 = geo.fixed_ref = true;
   geo.waves = 4;
   geo.rows = 128;
   if (a->head_dim == 64 && (prefix_causal || causal_q1)) {
@@ -418,8 +419,13 @@ int launch_fwd(const chia_attn_args* a, float* lse, void* stream) {
   // Softcap softmax on the one-block core: weights against a fixed reference
   // when cap log2 e <= 78 (cap <= 54), which keeps every weight normal
   // (attn_fwd_q1_kernel.h); north star 208.7 -> 200.6 us, headline 66.7 ->
-  // 62.7 us against the running max.
-  const bool cap_fixed = sp.softcap && a->norm == CHIA_ATTN_NORM_SOFTMAX && a->softcap * kLog2e <= 78.0f;
+  // 62.7 us against the running max.  Only where plan_geometry names that core
+  // by itself (head_dim 128, and at 64 banded masks, prefixes and large causal
+  // grids): grids that come from the paired core keep its running max, against
+  // which a row's largest weight is 1 and not rounded to bf16 (B1 H8 S512 D64,
+  // error against float64 0.00198; with the fixed reference 0.00211).
+  const bool cap_fixed =
+      geo.fixed_ref && sp.softcap && a->norm == CHIA_ATTN_NORM_SOFTMAX && a->softcap * kLog2e <= 78.0f;
   const int norm = (int)a->norm, which = norm + kNorms * geo.shape;
   KernelFn fn;
   if (!geo.q1)

@@ -450,3 +450,52 @@ def test_key_groups(name, B, H, S, D, kw):
         ref = oracle.attention_ref(*(t[b:b + 1, h:h + 1] for t in (q, k, v)), **part)
         res = gate.north_star_gate(ref, o[b:b + 1, h:h + 1], scale_aware=kw.get("norm", "softmax") != "softmax")
         assert res.ok, (name, b, h, res.status, res.stats)
+
+
+@pytest.mark.parametrize("cap", [30.0, 50.0])
+@pytest.mark.parametrize("name,B,H,S,causal", [
+    ("one_block", 1, 4, 64, True), ("four_groups", 1, 8, 512, True), ("two_groups", 2, 12, 1001, False),
+    ("full_rows", 2, 16, 1500, False), ("packed", 0, 4, 700, True)], ids=lambda x: x if isinstance(x, str) else "")
+def test_softcap_largest_weight_is_exact(name, B, H, S, causal, cap):
+    """Softcap softmax at head dim 64 on the grids without the fixed reference: a row's largest
+    weight is 1, without a rounding of its own.
+
+    Every row has two scores, 0 (odd keys) and s > 0 (even keys), with e^-s within 2^-12 of a
+    bf16 value, so against the row's max both weights are (nearly) bf16 numbers, and the ratio
+    of the two sums is off by 2^-12 and the fp32 exponents' error (below 2^-14).  A reference
+    that is not the row's max rounds both weights by up to 2^-8.  With o = w1 - c w0 (w1, w0
+    the weights' shares): |do| <= (1 + c) w1 w0 |d ratio| + the rounding of o to bf16, 8
+    significant bits: 2^-8 |o|."""
+    from chia_proj_amd import attention_varlen
+
+    _say(f"[parity] softcap largest weight {name} cap={cap}")
+    D = 64
+    alpha = (torch.arange(1, 60 * 256) / 256).to(torch.bfloat16).unique().double()
+    ratio = torch.exp(-cap * torch.tanh(alpha / math.sqrt(D) / cap))
+    near = (ratio / ratio.float().to(torch.bfloat16).double() - 1).abs() <= 2.0 ** -12
+    alpha = alpha[near & (ratio > 1 / 16)]
+    n_b = max(B, 1)
+    g = torch.Generator("cpu").manual_seed(S + H)
+    a = alpha[torch.randint(len(alpha), (n_b, H, S), generator=g)]
+    even = (torch.arange(S) % 2 == 0).double()
+    c = torch.exp2(torch.linspace(0, 3, D)).to(torch.bfloat16).double()
+    q, k, v = (torch.zeros(n_b, H, S, D, dtype=torch.float64) for _ in range(3))
+    q[..., 0] = a
+    k[..., 0] = even
+    v += even[:, None] - (1 - even)[:, None] * c
+    q, k, v = (t.to(torch.bfloat16).to(DEV) for t in (q, k, v))
+    kw = dict(causal=causal, softcap=cap)
+    if B == 0:  # two sequences of an even number of tokens, packed
+        cu = torch.tensor([0, 300, S], dtype=torch.int32, device=DEV)
+        o = attention_varlen(*(t[0].transpose(0, 1).contiguous() for t in (q, k, v)), cu, **kw).transpose(0, 1)[None]
+        seen = torch.cat([torch.arange(300), torch.arange(S - 300)]) + 1
+    else:
+        o = attention(q, k, v, **kw)
+        seen = torch.arange(S) + 1 if causal else torch.full((S,), S)
+    n1, n0 = ((seen + 1) // 2).double(), (seen // 2).double()
+    r = torch.exp(-cap * torch.tanh(a / math.sqrt(D) / cap))
+    w1 = (n1 / (n1 + n0 * r))[..., None]
+    ref = w1 - (1 - w1) * c
+    bound = (1 + c) * w1 * (1 - w1) * (2.0 ** -12 + 2.0 ** -14) + (2.0 ** -8 + 2.0 ** -20) * ref.abs() + 2.0 ** -20
+    err = (o.double().cpu() - ref).abs()
+    assert bool((err <= bound).all()), (name, float((err / bound).max()), float((err > bound).double().mean()))

@@ -767,8 +767,7 @@ def attention_varlen(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_seqle
     if needs_grad or torch.compiler.is_compiling():
         if out is not None:
             raise ValueError("out= is not supported when q, k or v requires grad or under torch.compile")
-        if (not torch.compiler.is_compiling() and plain_eager(q, k, v) and q.dim() == 3
-                and type(cu_seqlens) is torch.Tensor and cu_seqlens.is_cuda):
+        if not torch.compiler.is_compiling() and plain_eager(q, k, v, cu_seqlens) and q.dim() == 3:
             return eager_fwd_varlen(q, k, v, cu_seqlens, max_seqlen, _device_params(params, q))
         return _op_forward_varlen(q, k, v, cu_seqlens, max_seqlen, params)[0]
     if isinstance(q, torch.Tensor) and q.dim() == 3 and q.shape[0] == 0:

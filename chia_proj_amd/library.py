@@ -84,19 +84,33 @@ def _setup_context(ctx, inputs, output):
     ctx.set_materialize_grads(False)  # no zero-filled gradient for the unused lse
 
 
-def _traced(do: Tensor) -> bool:
-    """torch.compile, make_fx / AOTAutograd (a dispatch mode is active), or fake / meta
-    tensors: the backward is the registered operator, one node of the graph.  Eager on
-    the GPU it is the same implementation without a second operator dispatch."""
+_DK = torch._C.DispatchKey
+# The dispatch keys of a CUDA tensor whose memory holds its values.
+_PLAIN_KEYS = (torch._C.DispatchKeySet(_DK.CUDA).add(_DK.ADInplaceOrView).add(_DK.AutogradCUDA)
+               .add(_DK.AutocastCUDA))
+
+
+def _holds_values(t: Tensor) -> bool:
+    """False for tensors that torch's dispatch resolves before an operator reads them: batched
+    ones (vmap, is_grads_batched), negated views, zeros without memory, tensors of another
+    device.  Most of them are a plain torch.Tensor on a CUDA device by type."""
+    return torch._C._dispatch_keys(t) == _PLAIN_KEYS
+
+
+def _traced(do: Tensor, *saved: Tensor) -> bool:
+    """torch.compile, make_fx / AOTAutograd (a dispatch mode is active), fake / meta tensors,
+    or ones without values of their own: the backward is the registered operator, one node
+    of the graph.  Eager on the GPU it is the same implementation without a second operator
+    dispatch."""
     return (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0
-            or type(do) is not torch.Tensor or do.device.type != "cuda")
+            or type(do) is not torch.Tensor or not all(map(_holds_values, (do, *saved))))
 
 
 def _backward(ctx, do, _dlse):
     q, k, v, o, lse = ctx.saved_tensors
     if do is None:
         return (None,) * (3 + len(ctx.rest))
-    if _traced(do):
+    if _traced(do, q, k, v):
         dq, dk, dv = torch.ops.chia_attn.bwd(do, q, k, v, o, lse, *ctx.rest)
     else:
         from .attention import run_backward
@@ -134,12 +148,13 @@ _PLAIN_TYPES = (Tensor, torch.nn.Parameter)
 
 
 def plain_eager(*tensors) -> bool:
-    """True when nothing can observe whether the operator itself was dispatched: plain
-    CUDA tensors, no dispatch or function mode (tracing, FakeTensor, profiling
-    modes), no functorch transform (vmap, grad, jvp), no forward-mode level and no
-    TorchScript tracing."""
+    """True when the operator's dispatch would do nothing but call the implementation:
+    plain CUDA tensors that hold their values, no dispatch or function mode (tracing,
+    FakeTensor), no functorch transform (vmap, grad, jvp), no forward-mode level and no
+    TorchScript tracing.  (A profiler's trace shows such a call as the autograd function
+    below and not as chia_attn::fwd.)"""
     for t in tensors:
-        if type(t) not in _PLAIN_TYPES or not t.is_cuda:
+        if type(t) not in _PLAIN_TYPES or not _holds_values(t):
             return False
     return (torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
             and not torch._C._are_functorch_transforms_active()
@@ -233,7 +248,7 @@ def _backward_varlen(ctx, do, _dlse):
         return (None,) * (4 + len(ctx.rest))
     # grad mode is on here only under create_graph=True: the operator, which has no
     # second derivative, then refuses one instead of leaving it out of a sum
-    if _traced(do) or torch.is_grad_enabled():
+    if _traced(do, q, k, v) or torch.is_grad_enabled():
         dq, dk, dv = torch.ops.chia_attn.bwd_varlen(do, q, k, v, o, lse, cu_seqlens, *ctx.rest)
     else:
         from .attention import run_backward_varlen

@@ -300,3 +300,31 @@ def test_packed_second_derivative_is_refused():
         assert torch.equal(a, b)
     with pytest.raises(RuntimeError):
         (got[0].float().sum() + ts[0].float().sum()).backward()
+
+
+@pytest.mark.parametrize("packed", [False, True])
+def test_batched_and_negated_gradients(packed):
+    """Gradients and inputs that are plain CUDA tensors by type but whose memory does not hold
+    their values (a batch of gradients, is_grads_batched; negated views) meet the operator,
+    which torch calls once per gradient or with the values resolved."""
+    from chia_proj_amd import attention_varlen
+
+    _say(f"[lib] batched gradients packed={packed}")
+    cu = torch.tensor([0, 130, 300], dtype=torch.int32, device=DEV)
+    ts = _qkv(1, 4, 2, 300, 64, seed=12)
+    if packed:
+        ts = tuple(t[0].transpose(0, 1).contiguous() for t in ts)
+    ts = tuple(t.requires_grad_(True) for t in ts)
+    o = attention_varlen(*ts, cu, 170, causal=True) if packed else attention(*ts, causal=True)
+    g = torch.Generator("cpu").manual_seed(13)
+    dos = torch.randn(3, *o.shape, generator=g).to(torch.bfloat16).to(DEV)
+    want = [torch.autograd.grad(o, ts, do, retain_graph=True) for do in dos]
+    negated = torch.autograd.grad(o, ts, torch._neg_view(-dos[0]), retain_graph=True)
+    assert all(torch.equal(a, b) for a, b in zip(negated, want[0]))
+    got = torch.autograd.grad(o, ts, dos, is_grads_batched=True)
+    for i, a in enumerate(got):
+        assert torch.equal(a, torch.stack([w[i] for w in want]))
+    ns = tuple(torch._neg_view(-t.detach()).requires_grad_(True) for t in ts)  # negated inputs
+    on = attention_varlen(*ns, cu, 170, causal=True) if packed else attention(*ns, causal=True)
+    assert torch.equal(on, o)
+    assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(on, ns, dos[0]), want[0]))

@@ -97,12 +97,14 @@ def _holds_values(t: Tensor) -> bool:
     return torch._C._dispatch_keys(t) == _PLAIN_KEYS
 
 
-def _traced(do: Tensor, *saved: Tensor) -> bool:
+def _by_operator(do: Tensor, *saved: Tensor) -> bool:
     """torch.compile, make_fx / AOTAutograd (a dispatch mode is active), fake / meta tensors,
     or ones without values of their own: the backward is the registered operator, one node
-    of the graph.  Eager on the GPU it is the same implementation without a second operator
-    dispatch."""
-    return (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0
+    of the graph.  So it is under create_graph=True, the one time that grad mode is on here:
+    the operator has no second derivative and refuses one, where gradients without a graph
+    would leave it out of a sum in silence.  Otherwise, eager on the GPU, it is the same
+    implementation without a second operator dispatch."""
+    return (torch.is_grad_enabled() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0
             or type(do) is not torch.Tensor or not all(map(_holds_values, (do, *saved))))
 
 
@@ -110,7 +112,7 @@ def _backward(ctx, do, _dlse):
     q, k, v, o, lse = ctx.saved_tensors
     if do is None:
         return (None,) * (3 + len(ctx.rest))
-    if _traced(do, q, k, v):
+    if _by_operator(do, q, k, v):
         dq, dk, dv = torch.ops.chia_attn.bwd(do, q, k, v, o, lse, *ctx.rest)
     else:
         from .attention import run_backward
@@ -246,9 +248,7 @@ def _backward_varlen(ctx, do, _dlse):
     q, k, v, o, lse, cu_seqlens = ctx.saved_tensors
     if do is None:
         return (None,) * (4 + len(ctx.rest))
-    # grad mode is on here only under create_graph=True: the operator, which has no
-    # second derivative, then refuses one instead of leaving it out of a sum
-    if _traced(do, q, k, v) or torch.is_grad_enabled():
+    if _by_operator(do, q, k, v):
         dq, dk, dv = torch.ops.chia_attn.bwd_varlen(do, q, k, v, o, lse, cu_seqlens, *ctx.rest)
     else:
         from .attention import run_backward_varlen

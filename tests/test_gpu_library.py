@@ -302,6 +302,20 @@ def test_packed_second_derivative_is_refused():
         (got[0].float().sum() + ts[0].float().sum()).backward()
 
 
+def test_second_derivative_is_refused():
+    """As test_packed_second_derivative_is_refused, for attention()."""
+    _say("[lib] create_graph")
+    ts = _qkv(1, 2, 2, 96, 64, seed=4, grad=True)
+    o = attention(*ts, causal=True)
+    do = torch.ones_like(o)
+    want = torch.autograd.grad(o, ts, do, retain_graph=True)
+    got = torch.autograd.grad(o, ts, do, create_graph=True)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    with pytest.raises(RuntimeError):
+        (got[0].float().sum() + ts[0].float().sum()).backward()
+
+
 @pytest.mark.parametrize("packed", [False, True])
 def test_batched_and_negated_gradients(packed):
     """Gradients and inputs that are plain CUDA tensors by type but whose memory does not hold

@@ -17,14 +17,6 @@
 
 namespace chia {
 
-using KernelFn = void (*)(FwdParams);
-KernelFn select_kernel_d64(int waves, int norm, bool alibi, bool softcap);
-KernelFn select_q1_kernel_d64(int which, bool alibi, bool softcap, bool cap_fixed);
-KernelFn select_kernel_d128(int norm);
-KernelFn select_q1_kernel_d128(int which, bool alibi, bool softcap, bool cap_fixed);
-KernelFn select_q1_split_kernel_d128(int norm, bool alibi, bool softcap, bool cap_fixed);
-BwdKernels select_bwd_kernels_d64(int norm, bool alibi, bool softcap);
-BwdKernels select_bwd_kernels_d128(int norm, bool alibi, bool softcap);
 Fp8KernelFn select_fp8_kernel(int head_dim, int format, int norm, bool alibi, bool softcap);
 
 namespace {

@@ -263,21 +263,6 @@ __device__ __forceinline__ uint32_t stage_behind(uint32_t cur) {
   return cur == 0 ? NS - 1 : cur - 1;
 }
 
-// Workgroup shapes of both kernels: wavefronts that own 32 rows (dQ) or 32 keys
-// (dK/dV) each, times groups that split the walk over the key (query) tiles.
-constexpr int kBwdSplits = 3;
-struct BwdSplit {
-  int own, groups;
-};
-constexpr BwdSplit kBwdSplit[kBwdSplits] = {{4, 1}, {4, 2}, {2, 4}};
-
-// Kernel set of one (head_dim, normaliser, ALiBi, softcap) instantiation.
-using BwdKernelFn = void (*)(BwdParams);
-struct BwdKernels {
-  BwdKernelFn dq[kBwdSplits];
-  BwdKernelFn dkdv[kBwdSplits][2];  // [split][1: a K/V group's heads differ in scale]
-};
-
 // do . o over the 8 DK bf16 values of one lane's half row (chunks 16 kk + 8 lh
 // of the dQ kernel's register layout), in fp32.
 template <int DK>

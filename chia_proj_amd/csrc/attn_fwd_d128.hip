@@ -7,8 +7,6 @@
 
 namespace chia {
 
-using KernelFn = void (*)(FwdParams);
-
 KernelFn select_kernel_d128(int norm) {
   if (norm == NORM_SIGMOID) return attn_fwd_kernel<128, 4, NORM_SIGMOID, false, false>;
   if (norm == NORM_RELU) return attn_fwd_kernel<128, 4, NORM_RELU, false, false>;

@@ -5,8 +5,6 @@
 
 namespace chia {
 
-using KernelFn = void (*)(FwdParams);
-
 template <int NORM, bool AL, bool SC>
 static KernelFn inst() {
   return attn_fwd_kernel<64, 4, NORM, AL, SC>;

@@ -67,6 +67,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "launch_shapes.h"
 #include "lds_layout.h"
 #include "mask.h"
 
@@ -78,9 +79,6 @@ typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 typedef short i16x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) i16x4_t lds_i16x4_t;
-
-enum Norm : int { NORM_SOFTMAX = 0, NORM_SIGMOID = 1, NORM_RELU = 2 };
-constexpr int kNorms = 3;
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
@@ -181,11 +179,6 @@ __device__ __forceinline__ SeqSpan seq_span(const int32_t* cu_seqlens, int b, in
   }
   return s;
 }
-
-// Workgroup shapes of the one-block core: 128 rows by four wavefronts, the
-// same with two groups splitting a zigzag pair (head_dim 128), 128 rows by two
-// groups of four wavefronts that split the keys, 64 rows by four groups of two.
-enum Q1Shape : int { Q1_ONE = 0, Q1_ZIGZAG2 = 1, Q1_KEYS2 = 2, Q1_KEYS4 = 3 };
 
 // Waves per SIMD the register budget targets: two at head_dim 64 (the
 // hardware then overlaps one wave's softmax with the other's MFMAs), one at

@@ -6,8 +6,6 @@
 
 namespace chia {
 
-using KernelFn = void (*)(FwdParams);
-
 template <int NORM, bool AL, bool SC, int NG, int RW, int KG, bool CAPFIX = false>
 static KernelFn inst_q1() {
   return attn_fwd_q1_kernel<64, NORM, AL, SC, NG, CAPFIX, RW, KG>;
@@ -29,7 +27,6 @@ static KernelFn select_shape(int norm, bool alibi, bool softcap, bool cap_fixed)
   return table[norm][alibi ? 1 : 0][softcap ? 1 : 0];
 }
 
-// `which`: normaliser + kNorms times the shape (Q1Shape).
 KernelFn select_q1_kernel_d64(int which, bool alibi, bool softcap, bool cap_fixed) {
   const int norm = which % kNorms;
   switch (which / kNorms) {

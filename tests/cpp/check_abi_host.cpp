@@ -1,6 +1,6 @@
 // Host-side checks of the C ABI (include/chia_attn.h), built with
 // AddressSanitizer and UndefinedBehaviorSanitizer on the host code by
-// tests/test_sanitized_host.py.  Nothing here launches a kernel or needs a
+// tests/test_host_sanitized.py.  Nothing here launches a kernel or needs a
 // GPU: the checks cover the entry points that run on the host alone.
 //   * status strings, versioning;
 //   * argument validation of chia_attn_fwd, _fwd_lse, _bwd, _bwd_noalloc and
@@ -18,26 +18,20 @@
 #include <vector>
 
 #include "chia_attn.h"
+#include "launch_shapes.h"
 
 // The library's kernel selectors live in the kernel translation units, which
 // this host-only build does not link: no call below reaches a launch.
 namespace chia {
-struct FwdParams;
-struct BwdParams;
 struct Fp8Params;
-using KernelFn = void (*)(FwdParams);
-using BwdKernelFn = void (*)(BwdParams);
 using Fp8KernelFn = void (*)(Fp8Params);
-struct BwdKernels {
-  BwdKernelFn stats, dq, dkdv;
-};
 KernelFn select_kernel_d64(int, int, bool, bool) { return nullptr; }
 KernelFn select_q1_kernel_d64(int, bool, bool, bool) { return nullptr; }
 KernelFn select_kernel_d128(int) { return nullptr; }
 KernelFn select_q1_kernel_d128(int, bool, bool, bool) { return nullptr; }
 KernelFn select_q1_split_kernel_d128(int, bool, bool, bool) { return nullptr; }
-BwdKernels select_bwd_kernels_d64(int, bool, bool) { return BwdKernels{nullptr, nullptr, nullptr}; }
-BwdKernels select_bwd_kernels_d128(int, bool, bool) { return BwdKernels{nullptr, nullptr, nullptr}; }
+BwdKernels select_bwd_kernels_d64(int, bool, bool) { return BwdKernels{}; }
+BwdKernels select_bwd_kernels_d128(int, bool, bool) { return BwdKernels{}; }
 Fp8KernelFn select_fp8_kernel(int, int, int, bool, bool) { return nullptr; }
 }  // namespace chia
 

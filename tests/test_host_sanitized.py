@@ -35,7 +35,8 @@ def test_abi_host_code_under_sanitizers(tmp_path):
                     *HOST_SANITIZE, f"-I{inc}", f"-I{csrc}", "-c", str(csrc / "attn_api.hip"), "-o", str(api)],
                    check=True, capture_output=True)
     subprocess.run([str(CLANG), "-std=c++17", "-O1", "-g", "-fsanitize=address,undefined",
-                    "-fno-sanitize-recover=all", f"-I{inc}", "-c", str(ROOT / "tests" / "cpp" / "check_abi_host.cpp"),
+                    "-fno-sanitize-recover=all", f"-I{inc}", f"-I{csrc}", "-c",
+                    str(ROOT / "tests" / "cpp" / "check_abi_host.cpp"),
                     "-o", str(drv)], check=True)
     subprocess.run([str(CLANG), "-fsanitize=address,undefined", str(drv), str(api), "-o", str(exe),
                     f"-L{ROCM / 'lib'}", "-lamdhip64", f"-Wl,-rpath,{ROCM / 'lib'}"], check=True)

@@ -385,7 +385,7 @@ CHIA_HD MaskGeom residue_geom(const MaskSpec& m, int32_t r) {
 // 4 heads D128, 3174 + 3017 + 6 shorter sequences: 137.6 -> 56.0 us; 16 heads
 // D128, 1808 + 83 tokens: 58.3 -> 40.0.
 struct LaunchOrder {
-  int32_t shift, hx, hh, hs;
+  int32_t shift, hx, hh, hs, turn;  // turn: -1 (each rank begins one slice further on) or 0
   UDiv div_hx, div_hh;
 };
 struct SliceUnit {
@@ -395,11 +395,8 @@ struct SliceUnit {
 CHIA_HD SliceUnit rank_order(int x, const LaunchOrder& o, int n_units) {
   const int xcd = x & ((1 << o.shift) - 1), local = x >> o.shift;
   const int rank = udiv(local, o.div_hx);
-  int s = local - rank * o.hx;
-  if (o.hs > 0 && (o.hx & 1) == 0) {
-    s += rank;
-    s -= udiv(s, o.div_hx) * o.hx;
-  }
+  const int turned = local + (rank & o.turn);
+  const int s = turned - udiv(turned, o.div_hx) * o.hx;
   const int run = udiv(s, o.div_hh);
   return SliceUnit{run * o.hs + xcd * o.hh + (s - run * o.hh), n_units - 1 - rank};
 }
@@ -407,13 +404,14 @@ CHIA_HD SliceUnit rank_order(int x, const LaunchOrder& o, int n_units) {
 // The longest-first order over `slices` (batch, head, residue) slices
 // of `heads` heads, or the natural one when `on` is false.
 inline LaunchOrder launch_order(bool on, int64_t slices, int64_t heads, int64_t residues, bool packed) {
-  LaunchOrder o{0, 0, 1, 0, make_udiv(1), make_udiv(1)};
+  LaunchOrder o{0, 0, 1, 0, 0, make_udiv(1), make_udiv(1)};
   if (!on) return o;
   const bool per_seq = packed && residues == 1 && heads % 8 == 0;
   o.shift = slices % 8 == 0 ? 3 : 0;
   o.hx = (int32_t)(slices >> o.shift);
   o.hh = per_seq ? (int32_t)(heads / 8) : packed && o.shift ? 1 : o.hx;
   o.hs = per_seq ? (int32_t)heads : packed && o.shift ? 8 : 0;
+  o.turn = o.hs > 0 && o.hx % 2 == 0 ? -1 : 0;
   o.div_hx = make_udiv(o.hx);
   o.div_hh = make_udiv(o.hh);
   return o;

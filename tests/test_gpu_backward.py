@@ -120,17 +120,27 @@ def test_backward_d128_row_tile_edges(S, kw):
     _check(f"S={S} {kw}", grads, attention_grad_ref(q, k, v, do, **kw))
 
 
-# dK/dV workgroup shapes other than four key wavefronts in one group.  Few keys: two key
-# wavefronts and four query groups (lengths from one row tile, where groups stay empty, to
-# ragged tile counts; query heads of a K/V group that differ in scale).  256 workgroups of equal
-# walks: two query groups.
+# Workgroup shapes of dK/dV; each name begins with the one its size runs, which
+# test_launch_shapes.py checks against the launch rule.  four_groups: two key wavefronts and four
+# query groups (from few row tiles, where groups stay empty, to ragged tile counts; query heads
+# of a K/V group that differ in scale); two_groups: four key wavefronts and two query groups.
 SPLIT = [
-    *[(f"four_groups_S{S}_G{G}_d{D}", 1, 2 * G, 2, S, D, kw) for D in (64, 128) for G, kw in (
-        (1, dict(causal=True)), (3, dict(causal=True, head_scale=[0.5, 2.0, 1.0, 0.25, 1.5, 0.75])))
+    *[(f"{'four_groups' if S >= lo else 'one_group'}_S{S}_G{G}_d{D}", 1, 2 * G, 2, S, D, kw)
+      for D, G, lo in ((64, 1, 290), (64, 3, 65), (128, 1, 130), (128, 3, 33))
+      for kw in [dict(causal=True) if G == 1 else
+                 dict(causal=True, head_scale=[0.5, 2.0, 1.0, 0.25, 1.5, 0.75])]
       for S in (1, 33, 65, 130, 290)],
-    *[(f"two_groups_d{D}_{name}", 4, 16 * G, 16, 500, D, kw) for D in (64, 128) for G, name, kw in (
-        (1, "full", dict(causal=False)), (1, "sigmoid", dict(causal=False, norm="sigmoid", bias=-5.0)))],
+    *[(f"{'one_group' if D == 64 else 'two_groups'}_d{D}_{name}", 4, 16, 16, 500, D, kw) for D in (64, 128)
+      for name, kw in (("full", dict(causal=False)), ("sigmoid", dict(causal=False, norm="sigmoid", bias=-5.0)))],
     ("two_groups_gqa_window_d64", 4, 32, 16, 500, 64, dict(causal=False, window=300)),
+    ("two_groups_gqa_window_d128", 2, 16, 8, 1100, 128, dict(causal=True, window=200)),
+    *[(f"two_groups_S643_d64_{name}", 2, 12, 12, 643, 64, kw) for name, kw in (
+        ("full", dict(causal=False)), ("sigmoid", dict(causal=False, norm="sigmoid", bias=-5.0)),
+        ("relu", dict(causal=False, norm="relu", post_scale=0.01)))],
+    ("two_groups_causal_d64", 1, 32, 32, 643, 64, dict(causal=True)),
+    ("two_groups_causal_d128", 2, 32, 32, 257, 128, dict(causal=True)),
+    *[(f"two_groups_headscale_d{D}", 4, 16, 8, 513, D,
+       dict(causal=False, head_scale=[0.5 + 0.1 * h for h in range(16)])) for D in (64, 128)],
 ]
 
 
@@ -152,14 +162,22 @@ def test_backward_query_groups(name, B, H, Hkv, S, D, kw):
         _check(f"{name} b={b} hk={hk}", [grads[0][b:b + 1, hq]] + [g[b:b + 1, hk:hk + 1] for g in grads[1:]], refs)
 
 
-# dQ's key groups: four groups of 32-key tiles on two heads (from one tile to ragged counts), and
-# two groups where 64 to 128 blocks of equal, long walks leave CUs idle.
+# Workgroup shapes of dQ, named as SPLIT's: four_groups, 64 rows by four groups of 32-key tiles;
+# two_groups, 128 rows by two groups.
 DQ_SPLIT = [
-    *[(f"four_groups_{n}_S{S}_d{D}", 1, 2, S, D, kw) for D in (64, 128) for S in (40, 95, 129, 700)
+    *[(f"{'four_groups' if S >= lo else 'one_group'}_{n}_S{S}_d{D}", 1, 2, S, D, kw)
+      for D, lo in ((64, 193), (128, 385)) for S in (40, 95, 129, 193, 385, 700)
       for n, kw in (("causal", dict(causal=True)), ("prefix", dict(causal=True, prefix=50)),
                     ("alibi_softcap", dict(causal=True, softcap=20.0, alibi_slopes=[0.1, 0.01])))],
-    *[(f"two_groups_{n}_d{D}", 1, 16, 1000, D, kw) for D in (64, 128) for n, kw in (
+    *[(f"four_groups_{n}_S1000_d{D}", 1, 16, 1000, D, kw) for D in (64, 128) for n, kw in (
         ("full", dict(causal=False)), ("relu", dict(causal=False, norm="relu", post_scale=0.01)))],
+    *[(f"four_groups_window_S{S}_d{D}", 1, 2, S, D, dict(causal=True, window=200)) for D, S in ((64, 257), (128, 385))],
+    *[(f"two_groups_{n}_d{D}", 2, 12, 643, D, kw) for D in (64, 128) for n, kw in (
+        ("full", dict(causal=False)), ("relu", dict(causal=False, norm="relu", post_scale=0.01)),
+        ("sigmoid", dict(causal=False, norm="sigmoid", bias=-5.0)))],
+    *[(f"two_groups_{n}_S643_d{D}", 1, 32, 643, D, kw) for D in (64, 128) for n, kw in (
+        ("causal", dict(causal=True)), ("prefix", dict(causal=True, prefix=50)),
+        ("alibi_softcap", dict(causal=True, softcap=20.0, alibi_slopes=[0.01 * h for h in range(32)])))],
 ]
 
 

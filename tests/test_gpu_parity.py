@@ -420,20 +420,37 @@ def test_grouped_query_kv(name, H, Hkv, S, D, kw):
     assert res.ok, f"{name}: {res.status} {res.stats}"
 
 
-# Forwards whose workgroups split a block's keys between groups of wavefronts: small grids (64 rows
-# by four groups) from one row to ragged tile counts, where groups stay without a tile, and 192
-# blocks of full rows (128 rows by two groups).
+# Workgroup shapes of the one-block core; each name begins with the one its size runs, which
+# test_launch_shapes.py checks against the launch rule.  keys4: 64 rows by four key groups, from
+# where the rule begins to take it (causal: the first blocks have fewer tiles than groups) over
+# ragged tile counts; keys2: 128 rows by two groups; zigzag2: pairs of blocks split by two groups
+# (head dim 128); one: 128 rows, one group, at the lengths below those.
 KEY_GROUPS = [
-    *[(f"four_groups_S{S}_d{D}_{n}", 1, 2, S, D, kw) for D in (64, 128) for S in (1, 33, 65, 127, 129, 300, 511)
+    *[(f"{'keys4' if S >= lo else 'one'}_S{S}_d{D}_{n}", 1, 2, S, D, kw) for D, lo in ((64, 193), (128, 257))
+      for S in (1, 33, 65, 127, 129, 193, 257, 300, 511)
       for n, kw in (("causal", dict(causal=True)), ("full_relu", dict(causal=False, norm="relu", post_scale=0.01)))],
-    *[(f"four_groups_{n}_d{D}", 1, 3, 450, D, kw) for D in (64, 128) for n, kw in (
+    *[(f"{'one' if D == 128 and n in ('window', 'dilation') else 'keys4'}_{n}_d{D}", 1, 3, 450, D, kw)
+      for D in (64, 128) for n, kw in (
         ("softcap", dict(causal=True, softcap=30.0)), ("softcap80", dict(causal=True, softcap=80.0)),
         ("alibi", dict(causal=True, alibi_slopes=[0.5, 0.1, -0.05])), ("prefix", dict(causal=True, prefix=100)),
         ("sigmoid", dict(causal=False, norm="sigmoid", bias=-6.0)), ("window", dict(causal=True, window=200)),
         ("dilation", dict(causal=True, dilation=2)))],
-    *[(f"two_groups_{n}_d{D}", 2, 12, 1001, D, kw) for D in (64, 128) for n, kw in (
+    ("keys4_dilation_S513_d128", 1, 2, 513, 128, dict(causal=True, dilation=2)),
+    *[(f"keys2_{n}_d{D}", 2, 12, 1001, D, kw) for D in (64, 128) for n, kw in (
         ("full", dict(causal=False)), ("alibi", dict(causal=False, alibi_slopes=[0.01 * h for h in range(12)])),
-        ("sigmoid", dict(causal=False, norm="sigmoid", bias=-6.0)))],
+        ("sigmoid", dict(causal=False, norm="sigmoid", bias=-6.0)),
+        ("relu", dict(causal=False, norm="relu", post_scale=0.01)))],
+    *[(f"keys2_{n}_S385_d{D}", 4, 12, 385, D, kw) for D in (64, 128) for n, kw in (
+        ("causal", dict(causal=True)), ("prefix", dict(causal=True, prefix=100)),
+        ("causal_relu", dict(causal=True, norm="relu", post_scale=0.05)),
+        ("causal_alibi", dict(causal=True, alibi_slopes=[0.02 * h for h in range(12)])))],
+    *[(f"keys2_{n}_d{D}", B, H, S, D, kw) for D, B, H, S in ((64, 2, 32, 643), (128, 4, 12, 385))
+      for n, kw in (("softcap", dict(causal=True, softcap=30.0)), ("softcap80", dict(causal=True, softcap=80.0)))],
+    ("keys2_dilation_d64", 1, 32, 513, 64, dict(causal=True, dilation=2)),
+    ("keys2_dilation_d128", 2, 12, 777, 128, dict(causal=True, dilation=2)),
+    *[(f"zigzag2_{n}_d128", 4, 8, 1300, 128, kw) for n, kw in (
+        ("causal", dict(causal=True)), ("softcap", dict(causal=True, softcap=30.0)),
+        ("relu", dict(causal=True, norm="relu", post_scale=0.05)))],
 ]
 
 

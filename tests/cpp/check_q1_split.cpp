@@ -10,6 +10,10 @@
 //     barrier and waited for (vmcnt(0)), and a stage is refilled only after
 //     the barrier that follows its last read;
 //   * the merge buffer fits the workgroup's LDS.
+// And the key (query) groups of the one-block core and of both backward
+// kernels, for every step count a walk can have: step s computed once, by group
+// s % KG; every group passes the same barriers, so that the merge's two fall
+// together; the same two-stage DMA.
 // Build: g++ -std=c++17 -O2 -I chia_proj_amd/csrc tests/cpp/check_q1_split.cpp
 #include <cstdio>
 #include <vector>
@@ -139,6 +143,59 @@ void check_pair(const MaskGeom& g, int blk0, int blk1, const char* what) {
   CHECK((int)one.steps.size() == nsteps && (int)one.bars.size() == nsteps, "%s: one-group walk", what);
 }
 
+// One of KG groups over a walk of nsteps steps (>= 1), following the kernels'
+// statements: own steps 0, 1, ... are the walk's steps grp, grp + KG, ...
+Group walk_keys(int nsteps, int KG, int grp) {
+  int own = (nsteps - grp + KG - 1) / KG;  // s_hi, or ntiles in the backward
+  if (g_mistake == 5) own = nsteps / KG;
+  const int n_bar = (nsteps + KG - 1) / KG;
+  Group G;
+  std::vector<int> issued_at(n_bar + 1, -2), read_at_bar(n_bar + 1, -1);
+  int dma_next = 0, nb = 0;
+  for (; dma_next < NS - 1 && dma_next < own; ++dma_next) issued_at[dma_next] = -1;
+  for (int it = 0; it < n_bar; ++it) {
+    if (g_mistake == 6 && it >= own) break;  // before the step's barrier
+    G.bars.push_back('s');
+    ++nb;
+    if (dma_next < own) {
+      if (dma_next - NS >= 0)
+        CHECK(read_at_bar[dma_next - NS] >= 0 && read_at_bar[dma_next - NS] < nb, "stage of step %d refilled while read",
+              dma_next - NS);
+      issued_at[dma_next++] = nb;
+    }
+    if (it >= own) {
+      CHECK(it == n_bar - 1, "group %d of %d stops at step %d of %d", grp, KG, it, n_bar);
+      break;
+    }
+    CHECK(issued_at[it] != -2 && issued_at[it] < nb, "step %d read after barrier %d but issued at %d", it, nb, issued_at[it]);
+    read_at_bar[it] = nb;
+    G.steps.push_back(grp + it * KG);
+  }
+  CHECK(dma_next == imax32(own, 0), "group %d of %d issued %d of %d steps", grp, KG, dma_next, own);
+  G.bars.push_back('x');
+  G.bars.push_back('x');
+  return G;
+}
+
+long sweep_keys() {
+  long walks = 0;
+  for (int KG : {2, 4})
+    for (int nsteps = 1; nsteps <= 300; ++nsteps, ++walks) {
+      std::vector<int> seen(nsteps, 0);
+      const Group first = walk_keys(nsteps, KG, 0);
+      for (int grp = 0; grp < KG; ++grp) {
+        const Group g = walk_keys(nsteps, KG, grp);
+        CHECK(g.bars == first.bars, "%d steps: group %d of %d passes other barriers", nsteps, grp, KG);
+        for (int s : g.steps) {
+          CHECK(s < nsteps && s % KG == grp, "%d steps: group %d of %d computes step %d", nsteps, grp, KG, s);
+          if (s < nsteps) ++seen[s];
+        }
+      }
+      for (int s = 0; s < nsteps; ++s) CHECK(seen[s] == 1, "%d steps, %d groups: step %d computed %d times", nsteps, KG, s, seen[s]);
+    }
+  return walks;
+}
+
 }  // namespace
 
 long sweep() {
@@ -167,15 +224,15 @@ long sweep() {
 
 int main(int argc, char**) {
   if (argc > 1) {  // each planted mistake must be caught
-    for (g_mistake = 1; g_mistake <= 4; ++g_mistake) {
+    for (g_mistake = 1; g_mistake <= 6; ++g_mistake) {
       fails = 0;
-      const long n = sweep();
-      std::printf("planted mistake %d: %d violations over %ld pairs\n", g_mistake, fails, n);
+      const long n = g_mistake <= 4 ? sweep() : sweep_keys();
+      std::printf("planted mistake %d: %d violations over %ld %s\n", g_mistake, fails, n, g_mistake <= 4 ? "pairs" : "walks");
       if (fails == 0) return 1;
     }
     return 0;
   }
-  const long pairs = sweep();
+  const long pairs = sweep(), walks = sweep_keys();
   // LDS: the merge buffer (4 wavefronts x 64 lanes x (16 DB + 2) floats) within NG x NS stages
   for (int D : {64, 128}) {
     const int DB = D / 32, stage = 2 * BN * 2 * D;
@@ -185,6 +242,6 @@ int main(int argc, char**) {
     std::printf("%d violations\n", fails);
     return 1;
   }
-  std::printf("%ld zigzag pairs checked with two groups, 0 violations\n", pairs);
+  std::printf("%ld zigzag pairs and %ld group walks checked, 0 violations\n", pairs, walks);
   return 0;
 }

@@ -181,9 +181,9 @@ Geometry plan_geometry(const chia_attn_args* a, const MaskSpec& m, const ScorePa
   //     195.5 -> 172.1; with 32 slices slower (B2 H16 S4096 294.5 -> 312.9),
   //     and at 8192 rows slower or even (B1 H16 524.1 -> 578.2, B4 H16
   //     2023 -> 2032).
-  // Only where the longest-first order applies (it needs a multiple of 8
-  // slices and no packed sequences): in natural order the blocks' unequal work
-  // is not balanced.  Full rows keep the paired core (north star, temperature
+  // Not for packed sequences or slices that do not divide by 8, for which this
+  // schedule has no longest-first order (the launch has one: launch_order): in
+  // natural order the blocks' unequal work is not balanced.  Full rows keep the paired core (north star, temperature
   // 281.3 -> 302.6 us).
   bool causal_q1 = false;
   if (a->head_dim == 64 && geo.zigzag && !prefix_causal && !banded && a->norm == CHIA_ATTN_NORM_SOFTMAX &&
@@ -232,11 +232,12 @@ Geometry plan_geometry(const chia_attn_args* a, const MaskSpec& m, const ScorePa
 // times the shape's cost per step, plus its start-up (and merge) per round.
 // The paired core (full rows) and the zigzag pairs (causal rows, head_dim 128)
 // have equal walks and run in whole rounds of two workgroups per CU (one, with
-// two groups per pair).  The constants fit 690 timed shapes (1-4 sequences of
-// 128-8192 tokens, 4-32 heads, every mask and normaliser): 0.6 % above the best
-// candidate on average, and 1.37x (head_dim 64) and 1.22x (128) faster than
-// plan_geometry's schedule on drawn shapes, at most 3 % slower but for one 11 us
-// call.  For instance B1 H12 S3000 D64 causal: pairs 63 us, one block per
+// two groups per pair).  The constants were fit on drawn shapes (1-4 sequences
+// of 128-8192 tokens, 4-32 heads, every mask and normaliser).  On 800 others,
+// each candidate timed (profiles/launch_shape_times.csv), the choice is 2.2 %
+// (head_dim 64) and 2.7 % (128) above the best on average, 1.0 and 1.5 % without
+// the banded masks, and there 1.17x and 1.27x faster than plan_geometry's
+// schedule, at most 6 % slower.  For instance B1 H12 S3000 D64 causal: pairs 63 us, one block per
 // workgroup 49, KEYS2 37, KEYS4 28; B1 H32/16 S2500 D128 softcap 107, 77, 85,
 // 107; B4 H16 S2048 D64 causal 49, 48, 53, 63.
 struct StepCost {
@@ -293,6 +294,8 @@ Geometry launch_geometry(const chia_attn_args* a, const MaskSpec& m, const Score
       t = t > k * len * unit * loss ? t : k * len * unit * loss;
     }
     // softcap at head_dim 64: KEYS4's short steps hide its longer score chain
+    // (without the factors 2.3 % above the best and up to 16 % slower than the
+    // schedule on such shapes, with them 1.0 and 4 %)
     const double cap = !(d64 && sp.softcap) ? 1.0 : shape == Q1_KEYS2 ? 1.2 : shape == Q1_KEYS4 ? 0.8 : 1.0;
     return sc.per_step[shape] * cap * t + sc.start[shape] * std::fmax(1.0, n * waves / (kCUs * most));
   };
@@ -311,6 +314,9 @@ Geometry launch_geometry(const chia_attn_args* a, const MaskSpec& m, const Score
     keep = t + sc.start[Q1_ONE] < best;
     if (keep) best = t + sc.start[Q1_ONE];
   }
+  // Banded masks: their few steps leave the estimate little to go by, so key
+  // groups have to promise 15 % (at the same 1.0 as other masks some run 1.28x
+  // slower than one block per workgroup; so none does, at 2 % on average)
   if (!(packed && banded))
     for (int s : {Q1_KEYS2, Q1_KEYS4})
       if (const double t = shape_cost(s); t < (banded ? 0.85 : 1.0) * best) {
@@ -465,7 +471,10 @@ int64_t bwd_workspace(const chia_attn_args* a) {
 //   * the work of all of them spread evenly, or
 //   * the k-th round of CUs: k (P_k) where P_k is about the length of walk
 //     number 256 (k - 1) in falling order (the lengths taken as falling
-//     linearly from the longest), a workgroup of four wavefronts that is alone
+//     linearly from the longest; dK/dV of a window or block mask: as equal,
+//     since only the walks at a sequence's end are shorter.  B1 H32/16 S1165
+//     D128 block 256, 320 workgroups as {2, 4}: 71 us, where {4, 1} is 61; B3
+//     H24/12 S475 D64 window 256: 50 and 46), a workgroup of four wavefronts that is alone
 //     on its CU running at 1 / `alone` of the CU's rate,
 // times what the split costs per step (two groups: one workgroup per CU instead
 // of two, so start and end overlap less; four: each tile serves 64 rows or keys
@@ -473,25 +482,25 @@ int64_t bwd_workspace(const chia_attn_args* a) {
 struct SplitCost {
   double alone, per_step[kBwdSplits], start[kBwdSplits];
 };
-// dK/dV: fit on 110 drawn shapes (1-4 sequences of 128-4096 tokens, 1-32 K/V
-// heads, every mask): within 0.3 % of the best shape on average, never more
-// than 3 % above {4, 1}, which by itself was 21 % above the best (up to 1.9x:
-// B1 H32/8 S3000 D128 causal, dQ + dK/dV 561 us against 424 {4, 2} and 305
+// On 300 drawn shapes (1-4 sequences of 128-4096 tokens, 1-32 K/V heads, every
+// mask; profiles/launch_shape_times.csv, dQ + dK/dV), the choice of dK/dV is 0.2-0.3 %
+// above the best on average and at most 4 % above {4, 1}, which by itself is
+// 16 % (head_dim 64) and 23 % (128) above the best (up to 2x: B1 H32/8 S3000 D128 causal, dQ + dK/dV 561 us against 424 {4, 2} and 305
 // {2, 4}; B4 H16 S4096 D64 490 against 567 and 657).
 constexpr SplitCost kDkdvCost = {1.3, {1.0, 1.05, 1.6}, {4.0, 6.0, 6.0}};
-// dQ: fit on 200 drawn shapes, 0.1-0.2 % above the best; {4, 1} by itself 3 %
-// (dQ + dK/dV, up to 1.28x at head_dim 64 and 1.23x at 128).
+// dQ: 0.4-0.6 % above the best, at most 5 % above {4, 1}, which by itself is
+// 3 % above it (up to 1.28x).
 constexpr SplitCost kDqCostD64 = {1.5, {1.0, 0.95, 1.3}, {3.6, 7.0, 6.7}};
 constexpr SplitCost kDqCostD128 = {1.45, {1.0, 1.13, 2.1}, {4.1, 7.2, 6.3}};
 
-int pick_bwd_split(const SplitCost& sc, double slices, int32_t nblk, const double (&walk)[3]) {
+int pick_bwd_split(const SplitCost& sc, double slices, int32_t nblk, const double (&walk)[3], bool falling) {
   // the walks of the first, the middle and the last block
   const double longest = std::fmax(walk[0], std::fmax(walk[1], walk[2])), mean = 0.25 * (walk[0] + 2.0 * walk[1] + walk[2]);
   int best = 0;
   double best_cost = 0.0;
   for (int s = 0; s < kBwdSplits; ++s) {
     const BwdSplit sp = kBwdSplit[s];
-    const double unit = sp.own / 4.0, n = slices * nblk / unit, fall = 2.0 * (longest - mean) * kCUs / n;
+    const double unit = sp.own / 4.0, n = slices * nblk / unit, fall = falling ? 2.0 * (longest - mean) * kCUs / n : 0.0;
     double t = n * mean * unit / kCUs;
     for (int k = 1; k <= 8 && (k == 1 || (k - 1) * kCUs < n); ++k) {
       const double len = k * (longest - fall * (k - 1)) * unit * (k == 1 && sp.own * sp.groups == 4 ? sc.alone : 1.0);
@@ -513,7 +522,7 @@ int pick_dkdv_split(const MaskSpec& m, double slices, int64_t group, int32_t row
     const RowSpan r = query_range(g, blk * kBwdBlock, imin32(blk * kBwdBlock + kBwdBlock - 1, g.S - 1));
     return (double)group * (r.hi / row_tile - r.lo / row_tile + 1);
   };
-  return pick_bwd_split(kDkdvCost, slices, nblk, {walk(0), walk(nblk / 2), walk(nblk - 1)});
+  return pick_bwd_split(kDkdvCost, slices, nblk, {walk(0), walk(nblk / 2), walk(nblk - 1)}, m.hi >= kInf && m.blk == 0);
 }
 
 int pick_dq_split(const MaskSpec& m, double slices, bool d64) {
@@ -524,7 +533,7 @@ int pick_dq_split(const MaskSpec& m, double slices, bool d64) {
     return (double)(t.n_pre + t.n2);
   };
   return pick_bwd_split(d64 ? kDqCostD64 : kDqCostD128, slices, nblk,
-                        {walk(0), walk(nblk / 2), walk(nblk - 1)});
+                        {walk(0), walk(nblk / 2), walk(nblk - 1)}, true);
 }
 
 hipError_t launch(BwdKernelFn fn, int64_t grid, int threads, const BwdParams& p, hipStream_t stream) {

@@ -1,6 +1,8 @@
 """CPU checks of what chia_attn_fwd and chia_attn_bwd launch (tests/cpp/launch_shapes.cpp: the
 C ABI's own host code with the kernels replaced by tags and the launch call by a record)."""
+import csv
 import itertools
+import math
 import os
 import subprocess
 from pathlib import Path
@@ -114,3 +116,43 @@ def test_grids_cover_every_block(launches):
                 seen.add((per, D, split))
     assert {(c, D, 0) for c in ("one", "keys2", "keys4", "paired") for D in (64, 128)} <= seen
     assert {(per, D, s) for per in ("q", "kv") for D in (64, 128) for s in range(3)} <= seen
+
+
+TIMES = ROOT / "profiles" / "launch_shape_times.csv"  # (its columns: launch_shape_times.md)
+MASK_OF = {"causal": dict(causal=True), "full": dict(causal=False), "window256": dict(causal=True, window=256),
+           "local300": dict(causal=False, window=300), "block256": dict(causal=True, block=256),
+           "dil2": dict(causal=True, dilation=2), "prefix": dict(causal=True, prefix=256)}
+
+
+def test_rule_against_measured_times(launches):
+    """The launch rule on the shapes timed with every workgroup shape: on average at most 3 %
+    above the best one, and nowhere more than 6 % above one group per workgroup (forward: the
+    nominal schedule), which runs without a rule."""
+    rows = list(csv.DictReader(open(TIMES)))
+    calls = []
+    for r in rows:
+        kw = dict(MASK_OF[r["mask"]], norm=r["norm"])
+        if r["mod"]:
+            kw.update(softcap=40.0) if r["mod"] == "softcap" else kw.update(alibi_slopes=1)
+        calls.append((r["kind"], *(int(r[k]) for k in ("B", "H", "Hkv", "S", "D")), kw, 0))
+    above, slower = {}, []
+    for r, (kind, B, H, Hkv, S, D, kw, _), got in zip(rows, calls, launches(calls)):
+        t = [float(r[f"t{i}"]) if r[f"t{i}"] else math.inf for i in range(6)]
+        if kind == "fwd":
+            n, residues = _rows(S, kw)
+            pairs = B * H * residues * -(-(-(-n // 128)) // 2)
+            at = {"one": 0, "keys2": 1, "keys4": 2}.get(got[0], 3)
+            if got[0] == "one" and n > 128 and int(got[2]) == pairs:
+                at = 3  # pairs of blocks, one group
+            picks = [("fwd", t[at], min(t[:4]), t[3] if t[3] < math.inf else t[0])]
+        else:
+            picks = [("dq", t[int(got[0])], min(t[:3]), t[0]), ("dkdv", t[3 + int(got[3])], min(t[3:]), t[3])]
+        for name, pick, best, before in picks:
+            above.setdefault((name, D), []).append(math.log(pick / best))
+            if pick > 1.06 * before:
+                slower.append((r, name, got))
+    assert not slower, slower
+    for key, logs in above.items():
+        mean = math.exp(sum(logs) / len(logs))
+        print(key, len(logs), f"{mean:.4f}")
+        assert mean <= 1.03, (key, mean)

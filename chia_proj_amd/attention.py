@@ -66,6 +66,16 @@ def _head_key(vals: PerHead):
     return ("host", tuple(float(x) for x in vals))
 
 
+def _cached_vector(key) -> Optional[torch.Tensor]:
+    cached = _vec_cache.get(key)
+    if cached is not None:
+        try:
+            _vec_cache.move_to_end(key)  # the least recently used goes first
+        except KeyError:  # another thread has just dropped it
+            pass
+    return cached
+
+
 def _per_head_vector(vals: PerHead, heads: int, device: torch.device, name: str,
                      positive: bool, cache: bool = True) -> Optional[torch.Tensor]:
     """float32 [heads] device vector for a per-head parameter (cached for host values
@@ -80,7 +90,7 @@ def _per_head_vector(vals: PerHead, heads: int, device: torch.device, name: str,
             raise ValueError(f"{name} is on {t.device}, tensors are on {device}")
         return t.to(torch.float32).contiguous()
     if cache and type(vals) is tuple and len(vals) == heads:  # e.g. the variants' presets: seen before
-        cached = _vec_cache.get((name, device.index, vals))
+        cached = _cached_vector((name, device.index, vals))
         if cached is not None:
             return cached
     # host values: checked in Python (no tensor op, so fake-tensor tracing can run this)
@@ -101,14 +111,12 @@ def _per_head_vector(vals: PerHead, heads: int, device: torch.device, name: str,
     if not cache:
         return torch.tensor(host, dtype=torch.float32).to(device)  # a host constant, then a copy (traceable)
     key = (name, device.index, tuple(host))
-    cached = _vec_cache.get(key)
+    cached = _cached_vector(key)
     if cached is None:
         cached = torch.tensor(host, dtype=torch.float32).to(device)
         _vec_cache[key] = cached
         if len(_vec_cache) > _VEC_CACHE_MAX:
             _vec_cache.popitem(last=False)
-    else:
-        _vec_cache.move_to_end(key)
     return cached
 
 

@@ -2,6 +2,7 @@
 validation, and the no-fallback rule (no GPU calls are made here)."""
 import importlib
 import inspect
+import sys
 
 import pytest
 import torch
@@ -90,6 +91,21 @@ def test_cpu_tensors_are_rejected_not_computed():
 def test_validation_errors(bad, exc):
     with pytest.raises(exc):
         bad()
+
+
+def test_per_head_vectors_in_use_stay_cached(monkeypatch):
+    """The cache of device vectors drops the least recently used one; a tuple that finds its
+    vector at once counts as a use, so a model's own slopes survive a pass over many others."""
+    from collections import OrderedDict
+
+    core = sys.modules["chia_proj_amd.attention"]
+    monkeypatch.setattr(core, "_vec_cache", OrderedDict())
+    device, hot = torch.device("cpu"), (0.5, 0.25)
+    first = core._per_head_vector(hot, 2, device, "alibi_slopes", positive=False)
+    for i in range(2 * core._VEC_CACHE_MAX):
+        core._per_head_vector((1.0, float(i)), 2, device, "alibi_slopes", positive=False)
+        assert core._per_head_vector(hot, 2, device, "alibi_slopes", positive=False) is first, i
+    assert len(core._vec_cache) == core._VEC_CACHE_MAX
 
 
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):

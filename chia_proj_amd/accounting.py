@@ -7,7 +7,9 @@ Also reported: visited-tile FLOPs (tiles the kernel actually computes, at its
 wavefront tile of wave_m x block_n and at its workgroup tile of
 block_m x block_n) and dense-equivalent FLOPs 4 * D * S^2 * B * H.
 The visible-pair and tile counts come from chia_attn_plan, i.e. from the
-same mask functions the kernel runs.
+same mask functions the kernel runs.  The tile counts are its nominal
+schedule's, which the launches of the benchmark's headline and north-star
+shapes follow; small or unequal grids may take other blocks.
 """
 from __future__ import annotations
 

@@ -143,7 +143,8 @@ Geometry paired_geometry(const MaskSpec& m, int64_t batch, int64_t heads) {
 }
 
 // The nominal schedule, which chia_attn_plan describes and launch_geometry
-// starts from.  Head dim 64: the paired core, or for a
+// starts from (it launches no two-wavefront paired workgroups: they mark grids
+// too small for four).  Head dim 64: the paired core, or for a
 // window or block mask, causal rows with a prefix, and causal softmax on the
 // grids named below, the one-block core at four wavefronts per SIMD (north
 // star: local 53.2 -> 42.6 us, sliding window 53.1 -> 42.9, block-diagonal

@@ -223,14 +223,18 @@ typedef struct chia_attn_fp8_args {
 
 int chia_attn_fwd_fp8(const chia_attn_fp8_args* args, void* stream);
 
-/* Host-only statistics of the nominal schedule for `args` (no GPU call): the
- * launch may take another core or split the blocks' keys between groups of
- * wavefronts where the grid is small, over the same tiles.  Used by the
+/* Host-only statistics of the nominal schedule for `args` (no GPU call).  The
+ * launch takes another one where that is estimated to be faster (small grids
+ * and, at head_dim 64, causal rows): another core, other block heights, the
+ * keys of a block split between groups of wavefronts.  pairs_visible and
+ * residues hold for every launch; the blocks, wavefronts, workgroups and tile
+ * counts are the nominal schedule's only, and for some small head_dim 64 grids
+ * name two-wavefront workgroups that no kernel is built for.  Used by the
  * benchmark's FLOP accounting; the reference has no counterpart (its timer,
  * extra_bench.py:8-22, counts latency only). */
 typedef struct chia_attn_plan_info {
   int32_t block_m;          /* query rows a workgroup computes per KV tile: two row blocks
-                               (paired core), one (head_dim 128 one-block core) */
+                               (paired core), one (one-block core) */
   int32_t block_n;          /* keys per computed step: the 64-key KV tile (paired core) or
                                its 32-key halves (one-block core); tile counts below use it */
   int32_t wave_m;           /* rows of one computed sub-tile (32) */

@@ -118,6 +118,29 @@ def test_grids_cover_every_block(launches):
     assert {(per, D, s) for per in ("q", "kv") for D in (64, 128) for s in range(3)} <= seen
 
 
+def test_benchmark_shapes_launch_the_nominal_schedule(launches):
+    """The headline and north-star suites launch the schedule whose tile counts the FLOP
+    accounting quotes; a small grid need not."""
+    from chia_proj_amd import plan
+    from chia_proj_amd.accounting import core_plan_kwargs
+    from chia_proj_amd.workloads import headline_suite, north_star_suite
+
+    cases, plans, calls = [], [], []
+    for c in headline_suite() + north_star_suite():
+        params = dict(c.params, temperature=[1.0] * c.H) if c.temperature else c.params
+        kw = core_plan_kwargs(c.op, c.H, params)
+        plans.append(plan(batch=c.B, heads=c.H, seqlen=c.S, head_dim=c.D, **kw))
+        named = {k: kw[k] for k in ("norm", "causal", "window", "dilation", "block", "prefix", "softcap") if k in kw}
+        named.update({k: 1 for k, on in (("alibi_slopes", kw["alibi"]), ("head_scale", kw["head_scale"])) if on})
+        cases.append(c.name)
+        calls.append(("fwd", c.B, c.H, c.H, c.S, c.D, named, 0))
+    for name, p, got in zip(cases, plans, launches(calls)):
+        assert (got[0], int(got[1]), int(got[2])) == (
+            "one" if p["block_n"] == 32 else "paired", 64 * p["waves"], p["workgroups"]), (name, p, got)
+    small = plan(batch=1, heads=8, seqlen=512, head_dim=64, causal=True)
+    assert small["waves"] == 2 and launches([("fwd", 1, 8, 8, 512, 64, dict(causal=True), 0)])[0][0] == "keys4"
+
+
 TIMES = ROOT / "profiles" / "launch_shape_times.csv"  # (its columns: launch_shape_times.md)
 MASK_OF = {"causal": dict(causal=True), "full": dict(causal=False), "window256": dict(causal=True, window=256),
            "local300": dict(causal=False, window=300), "block256": dict(causal=True, block=256),

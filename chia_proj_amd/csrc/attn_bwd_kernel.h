@@ -93,7 +93,7 @@ struct BwdParams {
   MaskSpec mask;
   int32_t B, H, G;      // G: query heads per K/V head
   int32_t residues, SR;  // SR: stats row stride (residue 0 length, padded)
-  int32_t n_blk, n_wg;  // 128-row (or key) blocks per (b, head, residue 0); grid
+  int32_t n_blk, n_wg;  // blocks of the launched shape per (b, head, residue 0); grid
   UDiv div_blk, div_res, div_h, div_g, div_hk, div_dil;
   float scale, softcap, bias, post_scale;
   LaunchOrder order;  // the launched kernel's longest-first order (causal rows)
@@ -326,9 +326,9 @@ __global__ __launch_bounds__(64 * RW * KG, 2) void attn_bwd_dq_kernel(const BwdP
   char* const lds = lds_all + grp * (NS * STAGE_BYTES);  // the group's stages
   const int lq = lane & 31, lh = lane >> 5;
 
-  // workgroup -> (b, h, residue, 128-row block), heaviest blocks first
-  // (packed sequences of unequal length: round-robin over the XCDs, no remap)
-  // the query blocks with the most keys first
+  // workgroup -> (b, h, residue, block of BR rows).  Causal rows, packed or
+  // not: the query blocks with the most keys first (LaunchOrder).  Other packed
+  // sequences: in sequence order, round-robin over the XCDs, no remap
   int bhr, blk;
   if (p.order.hx > 0) {
     const SliceUnit su = rank_order((int)blockIdx.x, p.order, p.n_blk);
@@ -575,10 +575,9 @@ __global__ __launch_bounds__(64 * KW * QG, 2) void attn_bwd_dkdv_kernel(const Bw
   char* const lds = lds_all + grp * (NS * STAGE_BYTES);  // the group's stages
   const int lq = lane & 31, lh = lane >> 5;
 
-  // workgroup -> (b, K/V head, residue, 128-key block); low blocks (seen by
-  // the most rows under a causal mask) first
+  // workgroup -> (b, K/V head, residue, block of BK keys).  Causal rows, packed
+  // or not: the key blocks with the most queries, the first ones, first
   const int HK = p.H / p.G;
-  // the key blocks with the most queries (the first ones) first
   int bhr, blk = 0;
   int unit = -1;  // longest-first: blocks counted from the sequence's last one
   if (p.order.hx > 0) {

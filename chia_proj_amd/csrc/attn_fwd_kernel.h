@@ -16,9 +16,8 @@
 //     the pair is (2i, 2i+1);
 //   * the KV loop walks only the key tiles (BN = 64 keys) the mask can reach
 //     (prefix tiles + the band hull).  K and V tiles go from HBM straight into
-//     LDS with global_load_lds_dwordx4 (no VGPR staging) into four stages
-//     (two for 2-wavefront workgroups), up to three tiles ahead of the one
-//     computed, one barrier per step.
+//     LDS with global_load_lds_dwordx4 (no VGPR staging) into four stages, up
+//     to three tiles ahead of the one computed, one barrier per step.
 //     Each wavefront classifies the tile against its own rows and skips it
 //     (EMPTY), runs it unmasked (FULL) or with the per-element predicate
 //     (PARTIAL); band tiles inside precomputed ranges (fast_ranges) are known
@@ -200,10 +199,10 @@ struct IntTag {
 };
 
 // The software-pipelined run (below) is compiled where its registers fit
-// without spilling: 4 wavefronts, sigmoid / ReLU without a score modifier.
+// without spilling: sigmoid / ReLU without a score modifier.
 template <int D, int NW, int NORM, bool ALIBI, bool SOFTCAP>
 struct Pipelined {
-  static constexpr bool value = NW == 4 && NORM != NORM_SOFTMAX && !ALIBI && !SOFTCAP;
+  static constexpr bool value = NORM != NORM_SOFTMAX && !ALIBI && !SOFTCAP;
 };
 
 // 32-bit LDS address of a generic pointer into __shared__ memory.
@@ -308,11 +307,11 @@ __global__ __launch_bounds__(NW * 64, Occupancy<D>::value) void attn_fwd_kernel(
   constexpr bool kLazyMax = !ALIBI || kRev;  // softmax: the tile max only on demand
 
   constexpr bool kPipe = Pipelined<D, NW, NORM, ALIBI, SOFTCAP>::value;
-  // LDS stages: 4 for 4-wavefront workgroups (up to three tiles in flight;
-  // WIDE2 steps hold two), 2 for 2-wavefront ones.
-  constexpr int NS = NW == 4 ? 4 : 2;
+  // LDS stages: up to three tiles in flight; WIDE2 steps hold two.
+  static_assert(NW == 4, "four wavefronts per workgroup");
+  constexpr int NS = 4;
   static_assert((NS & (NS - 1)) == 0, "stage index is a mask");
-  constexpr bool kWide2 = NW == 4 && !kPipe;  // (the pipelined kernels keep their registers for the run)
+  constexpr bool kWide2 = !kPipe;  // (the pipelined kernels keep their registers for the run)
   __shared__ __attribute__((aligned(1024))) char lds[NS * STAGE_BYTES];
 
   const int tid = threadIdx.x;

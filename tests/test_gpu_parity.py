@@ -183,12 +183,12 @@ ALIBI_ORDER = [
 ]
 
 
-# Which core runs these shapes at head dim 64: B1 H2 (two slices) the paired core
-# on 2-wavefront workgroups; B4 H16 S2048 the paired core on 4-wavefront ones
-# (PAIR, WIDE and WIDE2 steps) for full rows, the one-block core for causal
-# softmax, prefixes, windows and blocks; B2 H16 S4096 (32 slices) the paired core
-# on 4-wavefront workgroups for causal rows too.  Head dim 128 runs the
-# one-block core throughout.
+# Which core runs these shapes at head dim 64 (test_launch_shapes.py checks it): B1 H2 (two
+# slices) the one-block core, four key groups (block256: one); B4 H16 S2048 the paired core (PAIR,
+# WIDE and WIDE2 steps) for full rows, the one-block core for causal softmax, prefixes, windows
+# and blocks; B2 H16 S4096 (exactly one round of pairs of whole tiles) the paired core for causal
+# rows too, but for softcap, which takes single blocks and the running max.  Head dim 128 runs
+# the one-block core throughout.
 PAIRED_CAUSAL = (2, 16, 4096)
 
 
@@ -224,7 +224,7 @@ def test_alibi_softmax_tile_order(name, kw, sign, shape, D):
 @pytest.mark.parametrize("name,kw,sign", [a for a in ALIBI_ORDER if a[0].startswith("causal")],
                          ids=[a[0] for a in ALIBI_ORDER if a[0].startswith("causal")])
 def test_alibi_softmax_tile_order_paired_causal(name, kw, sign):
-    """The same on causal rows of the paired core's 4-wavefront workgroups (B2 H16 S4096 D64)."""
+    """The same on causal rows of the paired core (B2 H16 S4096 D64)."""
     _alibi_order_case(name, kw, sign, PAIRED_CAUSAL, 64)
 
 
@@ -272,7 +272,8 @@ def test_softmax_rising_scores(name, kw, shape, D):
 @pytest.mark.parametrize("name,kw", [r for r in RISING if r[0] in ("causal", "softcap50", "headscale")],
                          ids=["causal", "softcap50", "headscale"])
 def test_softmax_rising_scores_paired_causal(name, kw):
-    """The same on causal rows of the paired core's 4-wavefront workgroups (B2 H16 S4096 D64)."""
+    """The same on causal rows of the paired core (B2 H16 S4096 D64; softcap50: single blocks of
+    the one-block core with the running max)."""
     _rising_case(name, kw, PAIRED_CAUSAL, 64)
 
 

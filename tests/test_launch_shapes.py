@@ -72,6 +72,24 @@ def test_group_cases_run_the_shapes_they_name(launches):
         assert case[0].startswith(SPLITS[int(got[0])]), (case, got)
 
 
+def test_adversarial_cases_run_the_cores_they_mean(launches):
+    """The shapes of test_softmax_rising_scores and test_alibi_softmax_tile_order at head dim 64."""
+    def core(shape, S, **kw):
+        B, H = shape
+        return launches([("fwd", B, H, H, S, 64, kw, 0)])[0][0]
+
+    B, H, S = test_gpu_parity.PAIRED_CAUSAL
+    for kw in (dict(), dict(alibi_slopes=1), dict(head_scale=1)):
+        assert core((B, H), S, causal=True, **kw) == "paired"
+        assert core((4, 16), 2048, causal=False, **kw) == "paired"
+        assert core((4, 16), 2048, causal=True, **kw) == "one"
+        assert core((1, 2), 512, causal=True, **kw) == core((1, 2), 700, causal=False, **kw) == "keys4"
+    assert core((B, H), S, causal=True, softcap=50.0) == "one"
+    for mask in (dict(causal=True, prefix=256), dict(causal=True, window=256), dict(causal=False, block=256)):
+        assert core((4, 16), 2048, **mask) == "one"
+        assert core((1, 2), 512, **mask) == ("one" if "block" in mask else "keys4")
+
+
 MASKS = [dict(causal=True), dict(causal=False), dict(causal=True, window=256), dict(causal=False, window=300),
          dict(causal=True, block=200), dict(causal=True, dilation=3), dict(causal=True, prefix=256)]
 SCORES = [dict(), dict(alibi_slopes=1), dict(softcap=30.0), dict(softcap=80.0)]

@@ -41,7 +41,8 @@ def log(*a):
 
 
 def kernel_name(op: str, B: int, H: int, S: int, D: int, params: dict) -> str:
-    """rocprofv3's name of the kernel instantiation a variant launches."""
+    """rocprofv3's name of the kernel instantiation a variant launches, where the launch follows
+    the nominal schedule (the headline and north-star suites)."""
     from chia_proj_amd import plan
     from chia_proj_amd.accounting import core_plan_kwargs
 
@@ -50,8 +51,9 @@ def kernel_name(op: str, B: int, H: int, S: int, D: int, params: dict) -> str:
     norm = {"softmax": 0, "sigmoid": 1, "relu": 2}[kw.get("norm", "softmax")]
     al = "true" if kw["alibi"] else "false"
     sc = "true" if kw.get("softcap", 0) else "false"
-    if p["block_n"] == 32:  # the head_dim 128 one-block core
-        return f"void chia::attn_fwd_q1_kernel<{D}, {norm}, {al}, {sc}>(chia::FwdParams)"
+    if p["block_n"] == 32:  # the one-block core: one group of four wavefronts, 128 rows
+        cap = "true" if norm == 0 and 0 < kw.get("softcap", 0) <= 54 else "false"  # the fixed reference
+        return f"void chia::attn_fwd_q1_kernel<{D}, {norm}, {al}, {sc}, 1, {cap}, 4, 1>(chia::FwdParams)"
     return f"void chia::attn_fwd_kernel<{D}, {p['waves']}, {norm}, {al}, {sc}>(chia::FwdParams)"
 
 

@@ -6,6 +6,8 @@ where a sweep row counts only if its status is "generalises".  Skipped where the
 reference tree is absent (it never travels to the GPU box)."""
 import csv
 import importlib.util
+import shutil
+import subprocess
 from pathlib import Path
 
 import pytest
@@ -60,3 +62,23 @@ def test_reference_suites_keep_the_reference_shape():
         assert [c.op for c in cases] == [c.op for c in reference_suite()]
         assert all((c.B, c.H, c.S, c.D) == (2, 32, S, 128) and c.params == {} for c in cases)
     assert reference_suite()[0].seed == 20262048  # the benchmark's draw is unchanged
+
+
+@pytest.mark.skipif(shutil.which("nm") is None, reason="nm not available")
+def test_kernel_names_are_the_librarys():
+    """The instantiation names that bench.py looks recorded HBM traffic up by are kernels of the
+    built library, as rocprofv3 prints them, and profiles/traffic.json records those names."""
+    from chia_proj_amd import _lib
+    from chia_proj_amd.workloads import headline_suite, north_star_suite
+
+    if not Path(_lib.LIB_PATH).exists():
+        pytest.skip("the library is not built")
+    out = subprocess.run(["nm", "-C", str(_lib.LIB_PATH)], capture_output=True, text=True, check=True).stdout
+    names = {line.split(" ", 2)[2] for line in out.splitlines() if "chia::attn_fwd" in line}
+    bench = _bench()
+    for suite, cases in (("headline", headline_suite()), ("northstar", north_star_suite())):
+        for c in cases:
+            params = dict(c.params, temperature=[1.0] * c.H) if c.temperature else c.params
+            name = bench.kernel_name(c.op, c.B, c.H, c.S, c.D, params)
+            assert name in names, (c.name, name)
+            assert bench.load_traffic(suite, c.op, name), (c.name, name)

@@ -159,7 +159,9 @@ def test_benchmark_shapes_launch_the_nominal_schedule(launches):
     assert small["waves"] == 2 and launches([("fwd", 1, 8, 8, 512, 64, dict(causal=True), 0)])[0][0] == "keys4"
 
 
-TIMES = ROOT / "profiles" / "launch_shape_times.csv"  # (its columns: launch_shape_times.md)
+# Measured times, us per call.  Forward: t0 one group, t1 keys2, t2 keys4, t3 the nominal schedule
+# where it has a kernel.  Backward (dQ + dK/dV): t0-t2 dQ's splits, t3-t5 dK/dV's.
+TIMES = ROOT / "profiles" / "launch_shape_times.csv"
 MASK_OF = {"causal": dict(causal=True), "full": dict(causal=False), "window256": dict(causal=True, window=256),
            "local300": dict(causal=False, window=300), "block256": dict(causal=True, block=256),
            "dil2": dict(causal=True, dilation=2), "prefix": dict(causal=True, prefix=256)}
